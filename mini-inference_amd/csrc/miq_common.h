@@ -212,7 +212,7 @@ struct Tuning {
   bool fp8_quant_rows_wg;     // MIQ_FP8_QUANT_ROWS_WG: one workgroup per row in fp8_quantize_rows
   bool moe_tiled;             // MIQ_MOE_TILED: the tiled expert kernels
   bool moe_four_waves;        // MIQ_MOE_WAVES=4: four-wavefront streaming expert workgroups
-  bool moe_no_lds_scales;     // MIQ_MOE_LDS_SCALES=0: per-k-step scale loads instead of LDS
+  bool moe_no_lds_scales;     // MIQ_MOE_LDS_SCALES=0: per-k-step scale loads
   bool moe_align_scan;        // MIQ_MOE_ALIGN_SCAN: the one-wavefront-per-expert align
   bool moe_align_launch;      // MIQ_MOE_ALIGN_LAUNCH: routed MoE entry points run moe_align
 };

@@ -384,14 +384,15 @@ constexpr int KIND_FP8 = 2;
 constexpr int kF8Steps = 2 * kMoeChunk;
 constexpr int kF8Row = kF8Steps * kStepK + 16;
 
-// SL (16-bit scales, at most kMoeLdsGroups groups per row, a multiple of 4): at the start
-// of an item each lane loads the scale and zero words of its row's groups 4 g .. 4 g + 3
-// with one 8-byte load each, and the wavefront keeps them in its LDS slice [tile][group]
-// [row] as (scale | zero << 16); a k-step then reads one LDS word per tile instead of
-// issuing two 4-byte global loads.
-constexpr int kMoeLdsGroups = 16;
-template <bool HZ>
-constexpr size_t kMoeScaleLdsPerWave = (size_t)2 * kMoeLdsGroups * kTile * (HZ ? 4 : 2);  // 2 tiles
+// SL (16-bit scales, at most kMoeRegGroups groups per row, a multiple of 4): at the start
+// of an item lane (r, g) loads the scale and zero words of row r's groups 4 g .. 4 g + 3 with
+// one 8-byte load each and keeps them in registers as (scale | zero << 16); a k-step of group
+// c takes its word from lane (r, c / 4) by ds_bpermute (no LDS storage) instead of issuing
+// two 4-byte global loads. An LDS table of the words instead took 16 KiB per eight-wavefront
+// workgroup with zero points, which left room for four-wavefront workgroups only (two
+// wavefronts per SIMD): OLMoE layer with zero points, 64 tokens, gate/up 37.4 -> 31.8 us and
+// down 25.9 -> 20.4 us (3.7 -> 4.3 and 2.8 -> 3.5 TB/s of weights).
+constexpr int kMoeRegGroups = 16;
 
 // eight-wavefront workgroups are held to 128 VGPRs (four wavefronts per SIMD, two
 // workgroups per CU; the routing code had taken the 8-bit down kernels to 132-140, one
@@ -471,9 +472,6 @@ moe_stream_kernel(MoeParams p, int blocks_per_tile, int run) {
   // maxima after them
   float* xsum = F8 ? reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(lds) + kTile * kF8Row)
                    : reinterpret_cast<float*>(lds + kTile * xstride);
-  // SL slice of this wavefront: (scale | zero << 16) words, or 16-bit scales without zero points
-  using ScEntry = std::conditional_t<HZ, uint32_t, uint16_t>;
-  ScEntry* scz = reinterpret_cast<ScEntry*>(xsum + kMoeChunk * kTile) + wv * (2 * kMoeLdsGroups * kTile);
   const int wbytes = (int)((int64_t)p.E * rows_per_expert * ldw);
   constexpr int esz = SD == MIQ_F32 ? 4 : 2;
   const int sbytes = (int)(((int64_t)p.E * rows_per_expert * ngroups * esz + 3) & ~3LL);
@@ -551,31 +549,37 @@ moe_stream_kernel(MoeParams p, int blocks_per_tile, int run) {
             wq[d + h][t][0] = *reinterpret_cast<const uint4*>(&v);
           }
         }
-        if (SL) continue;  // the item's scales are in LDS
+        if (SL) continue;  // the item's scales are in registers
         const int gi = soff[t] + kl / p.group_steps;  // (int4 only past here)
         const int so = ((gi * esz) & ~3 & keep) | (kOut & ~keep);
         sq[d][t] = __builtin_amdgcn_raw_buffer_load_b32(srs, so, 0, 0);
         zq[d][t] = HZ ? __builtin_amdgcn_raw_buffer_load_b32(zrs, so, 0, 0) : 0u;
       }
     };
-    // SL: this lane's 4 groups of each tile (loads past the row's groups return zeros)
-    uint32_t scw[NR][2], zcw[NR][2];
+    // SL: this lane's 4 groups of each tile (lanes past the row's groups hold zeros)
+    uint32_t scz[NR][4];
     if constexpr (SL) {
 #pragma unroll
       for (int t = 0; t < NR; ++t) {
         const int so = 4 * g < (int)ngroups ? (int)((soff[t] + 4 * g) * 2) : kOut;
         const auto vs = __builtin_amdgcn_raw_buffer_load_b64(srs, so, 0, 0);
-        scw[t][0] = vs[0];
-        scw[t][1] = vs[1];
+        uint32_t z0 = 0u, z1 = 0u;
         if (HZ) {
           const auto vz = __builtin_amdgcn_raw_buffer_load_b64(zrs, so, 0, 0);
-          zcw[t][0] = vz[0];
-          zcw[t][1] = vz[1];
-        } else {
-          zcw[t][0] = zcw[t][1] = 0u;
+          z0 = vz[0];
+          z1 = vz[1];
         }
+        scz[t][0] = (vs[0] & 0xffffu) | (z0 << 16);
+        scz[t][1] = (vs[0] >> 16) | (z0 & 0xffff0000u);
+        scz[t][2] = (vs[1] & 0xffffu) | (z1 << 16);
+        scz[t][3] = (vs[1] >> 16) | (z1 & 0xffff0000u);
       }
     }
+    // the (scale | zero << 16) word of group c (uniform) of this lane's row of tile t
+    auto group_word = [&](int t, int c) -> uint32_t {
+      const uint32_t lo = (c & 1) ? scz[t][1] : scz[t][0], hi = (c & 1) ? scz[t][3] : scz[t][2];
+      return (uint32_t)__builtin_amdgcn_ds_bpermute((r + 16 * (c >> 2)) * 4, (int)((c & 2) ? hi : lo));
+    };
 #pragma unroll
     for (int d = 0; d < D; ++d) request(d, d);
     // the tile's pairs (after the weight requests, which do not depend on them)
@@ -633,18 +637,6 @@ moe_stream_kernel(MoeParams p, int blocks_per_tile, int run) {
     int lpair[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) lpair[v] = MODE == MOE_DN && KIND == KIND_INT4 ? s_pair[g * 4 + v] : 0;
-    if constexpr (SL) {
-      // (only this wavefront reads its slice, in program order after these writes)
-#pragma unroll
-      for (int t = 0; t < NR; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t sw = scw[t][j >> 1], zw = zcw[t][j >> 1];
-          const uint32_t sh = (j & 1) ? sw >> 16 : sw & 0xffffu, zh = (j & 1) ? zw >> 16 : zw & 0xffffu;
-          if (4 * g + j < (int)ngroups) scz[(t * kMoeLdsGroups + 4 * g + j) * kTile + r] = (ScEntry)(sh | (zh << 16));
-        }
-    }
-
     uint4 wnext[NR];
     // Per quantization group, T = sum_k x (128 + u) + kXBias * sum_k x (MFMA chains and the
     // staged sums, which hold kXBias times the sum of x over each k-step), and
@@ -823,7 +815,7 @@ moe_stream_kernel(MoeParams p, int blocks_per_tile, int run) {
                 // one-step groups: chains from the step's bias and from zero; the group ends here
                 const int gi = soff[t] + c_grp;
                 uint32_t scw_l = 0;
-                if constexpr (SL) scw_l = scz[(t * kMoeLdsGroups + c_grp) * kTile + r];
+                if constexpr (SL) scw_l = group_word(t, c_grp);
                 const float sc = SL ? sd_to_f32<SD>(scw_l & 0xffffu) : word_to_f32<SD>(sq[d][t], gi);
                 f32x4 c0v = mfma(av[0], bv[0], xb);
                 f32x4 c1v = mfma(av[1], bv[1], z4);
@@ -848,7 +840,7 @@ moe_stream_kernel(MoeParams p, int blocks_per_tile, int run) {
               for (int t = 0; t < NR; ++t) {
                 const int gi = soff[t] + c_grp;
                 uint32_t scw_l = 0;
-                if constexpr (SL) scw_l = scz[(t * kMoeLdsGroups + c_grp) * kTile + r];
+                if constexpr (SL) scw_l = group_word(t, c_grp);
                 const float sc = SL ? sd_to_f32<SD>(scw_l & 0xffffu) : word_to_f32<SD>(sq[d][t], gi);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) acc[t][v] = __builtin_fmaf(sc, accg[t][v] + xsg[v], acc[t][v]);
@@ -923,13 +915,13 @@ void launch_stream_mode(const MoeParams& p, int grid, size_t lds, int blocks, in
     allow_max_dynamic_lds(reinterpret_cast<const void*>(&moe_stream_kernel<KIND, MODE, HZ, SD, G1, SL, NW>));
   });
   hipLaunchKernelGGL((moe_stream_kernel<KIND, MODE, HZ, SD, G1, SL, NW>), dim3(grid), dim3(NW * 64),
-                     lds + (SL ? NW * kMoeScaleLdsPerWave<HZ> : 0), st, p, blocks, run);
+                     lds, st, p, blocks, run);
 }
 
 // One GEMM of the layer: NW = 8 wavefronts (twice the weight rows per staged activation
 // tile, four wavefronts per SIMD) where the sizes divide and two such workgroups fit a CU's
-// LDS, else 4; int4 with 16-bit scales keeps the item's scales in LDS where a row's groups
-// fit. MIQ_MOE_WAVES=4 forces four wavefronts.
+// LDS, else 4; int4 with 16-bit scales keeps the item's scales in registers where a row's
+// groups fit. MIQ_MOE_WAVES=4 forces four wavefronts.
 template <int KIND, int MODE, bool HZ, int SD, bool G1>
 void launch_stream_gemm(const MoeParams& p, int max_tiles, hipStream_t st) {
   const size_t lds = KIND == KIND_FP8 ? (size_t)kTile * kF8Row + (size_t)kF8Steps * kTile * 4
@@ -937,11 +929,11 @@ void launch_stream_gemm(const MoeParams& p, int max_tiles, hipStream_t st) {
   const int K = MODE == MOE_GU ? p.H : p.I;
   const int ng = K / kStepK / p.group_steps;
   constexpr bool kSL16 = KIND == KIND_INT4 && SD != MIQ_F32;
-  const bool sl = kSL16 && ng % 4 == 0 && ng <= kMoeLdsGroups && !tuning().moe_no_lds_scales;
+  const bool sl = kSL16 && ng % 4 == 0 && ng <= kMoeRegGroups && !tuning().moe_no_lds_scales;
   const int per8 = MODE == MOE_GU ? 16 * 8 : 32 * 8;  // weight columns / rows of an 8-wavefront item
   const int nout = MODE == MOE_GU ? p.I : p.H;
   const bool w8 = !tuning().moe_four_waves && nout % per8 == 0 &&
-                  2 * (lds + (sl ? 8 * kMoeScaleLdsPerWave<HZ> : 0) + kMoeStaticLds) <= (size_t)160 * 1024;
+                  2 * (lds + kMoeStaticLds) <= (size_t)160 * 1024;
   const int blocks = nout / (w8 ? per8 : per8 / 2);
   // about two workgroups per CU, never more than the runs of items that could exist
   // runs of two items per workgroup where there are enough items for two workgroups per CU
