@@ -18,6 +18,7 @@
 
 #include <mutex>
 
+#include "fp8_split.h"
 #include "miq_common.h"
 
 namespace miq {
@@ -458,13 +459,17 @@ extern "C" int miq_fp8_gemm(const uint8_t* xq, const float* x_scale, const uint8
               "fp8_gemm: operands must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   uint16_t* yy = static_cast<uint16_t*>(y);
+  // kernels that address the operands through buffer descriptors take operands below 2 GiB
+  const bool buffers = !tuning().fp8_old && M * K < 0x7fffff00LL && N * K < 0x7fffff00LL;
   if (M >= 1024 && N % 192 == 0) {
-    // the large-tile kernel addresses the operands through buffer descriptors (< 2 GiB)
-    // and stores 16-byte pieces of y rows
-    if (!tuning().fp8_old && M * K < 0x7fffffffLL && N * K < 0x7fffffffLL && ldy % 8 == 0 &&
-        (reinterpret_cast<uintptr_t>(y) & 15) == 0)
+    // the large-tile kernel stores 16-byte pieces of y rows
+    if (buffers && ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0)
       return launch32<256, 192>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
     return launch<256, 192, 4, 2>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
+  }
+  if (buffers) {
+    const Fp8SplitPlan pl = fp8_split_plan(M, N, K);
+    if (pl.mt != 0) return fp8_split_launch(pl, xq, x_scale, wq, w_scale, yy, ldy, M, N, K, st);
   }
   return launch<128, 128, 2, 2>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
 }

@@ -1,0 +1,53 @@
+"""The split-K FP8 GEMM at the edges of its tiles, its K split and its dispatch range."""
+import pytest
+import torch
+
+from oracle import quant as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# (M, N, K): M around 16, 32 and 64 rows; N with a part tile (and not a multiple of 4 or 16);
+# one k-step, fewer k-steps than wavefronts and splits of unequal length; the sizes around
+# which the planner hands over to the 128 x 128 tiles, and the large-tile kernel's lower end
+SIZES = [(1, 16, 128), (1, 6144, 2560), (2, 20, 256), (15, 48, 384), (16, 2560, 9728), (17, 33, 640), (32, 80, 1152),
+         (33, 6144, 2560), (49, 130, 256), (64, 1008, 1024), (65, 2560, 4096), (129, 200, 896), (255, 19456, 256),
+         (257, 19456, 256), (300, 1024, 1024), (512, 6144, 640), (1023, 192, 384), (1024, 192, 384), (1025, 208, 384)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("pad", [0, 6])
+def test_fp8_gemm_tiles_and_splits(M, N, K, pad):
+    """fp32 products of exact e4m3 values in another order, then one rounding to bf16: within
+    half a bf16 ulp (8 significant bits: at most 2^-8 of the value) plus K * 2^-24 of the sum of |products|, which bounds
+    any order of fp32 additions. Output rows at a stride past N (pad, not a multiple of 4)
+    leave the padding alone."""
+    from kernels import _lib as L
+    print(f"[case] fp8 split M={M} N={N} K={K} pad={pad}", flush=True)
+    g = torch.Generator().manual_seed(M * 31 + N + K)
+    xq, xs = O.fp8_quantize_activation(torch.randn(M, K, generator=g).to(torch.bfloat16))
+    w = O.fp8_quantize((torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16))
+    xd, wd = xq.to(DEV), w["qweight"].to(DEV)
+    xsd, wsd = xs.reshape(-1).to(DEV), w["scale"].to(DEV)
+    y = torch.full((M, N + pad), 7.0, dtype=torch.bfloat16, device=DEV)
+    L.call("miq_fp8_gemm", L.ptr(xd), L.ptr(xsd), L.ptr(wd), L.ptr(wsd), L.ptr(y), N + pad, M, N, K, L.stream(y.device))
+    x64, w64 = xd.double(), wd.double()
+    s = xsd.double()[:, None] * wsd.double()[None, :]
+    want, mag = (x64 @ w64.t()) * s, (x64.abs() @ w64.abs().t()) * s
+    bound = (2.0 ** -8 + 2.0 ** -22) * want.abs() + K * 2.0 ** -24 * mag + 1e-30
+    assert ((y[:, :N].double() - want).abs() <= bound).all()
+    assert (y[:, N:] == 7.0).all()
+
+
+def test_fp8_gemm_repeats_bit_for_bit():
+    """The wavefronts' partial sums are added in a fixed order."""
+    from kernels import quant_ops as ops
+    print("[case] fp8 split repeat", flush=True)
+    g = torch.Generator().manual_seed(5)
+    xq, xs = O.fp8_quantize_activation(torch.randn(40, 2560, generator=g).to(torch.bfloat16))
+    w = O.fp8_quantize((torch.randn(6144, 2560, generator=g) * 0.02).to(torch.bfloat16))
+    args = [t.to(DEV) for t in (xq, xs, w["qweight"], w["scale"])]
+    first = ops.fp8_gemm(*args)
+    for _ in range(3):
+        assert torch.equal(ops.fp8_gemm(*args), first)
