@@ -170,6 +170,15 @@ int miq_fp8_gemm(const uint8_t* xq, const float* x_scale, const uint8_t* wq,
                  const float* w_scale, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K,
                  void* stream);
 
+/* Replaces FP8WeightAct.linear on a native device (fp8.py:48-61): miq_fp8_quantize_rows of x
+ * into the workspace, then miq_fp8_gemm, on one stream. x: [M, K] (x_dtype bf16/f16/f32, row
+ * stride ldx); the rest as those two. The workspace (miq_fp8_linear_workspace_bytes, 16-byte
+ * aligned) needs no initial value; calls that may overlap need one each. */
+size_t miq_fp8_linear_workspace_bytes(int64_t M, int64_t K);
+int miq_fp8_linear(const void* x, int x_dtype, int64_t ldx, const uint8_t* wq, const float* w_scale,
+                   void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, void* workspace,
+                   size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------ KV cache
  * Replaces KVCache._quantize + KVCache.write (engine/core/kv_cache.py:359-388) for one
  * layer and one of K or V: per (token, head) s = bf16(clamp(max|x| / qmax, 1e-8)),

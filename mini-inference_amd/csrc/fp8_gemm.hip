@@ -473,3 +473,20 @@ extern "C" int miq_fp8_gemm(const uint8_t* xq, const float* x_scale, const uint8
   }
   return launch<128, 128, 2, 2>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
 }
+
+extern "C" size_t miq_fp8_linear_workspace_bytes(int64_t M, int64_t K) {
+  return M < 1 || K < 1 ? 0 : (size_t)((M * K + 15) & ~15LL) + (size_t)M * sizeof(float);
+}
+
+extern "C" int miq_fp8_linear(const void* x, int x_dtype, int64_t ldx, const uint8_t* wq, const float* w_scale,
+                              void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+  MIQ_REQUIRE(M >= 1 && K >= 1, "fp8_linear: bad shape M=%lld K=%lld", (long long)M, (long long)K);
+  const size_t need = miq_fp8_linear_workspace_bytes(M, K);
+  MIQ_REQUIRE(workspace != nullptr && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0,
+              "fp8_linear: %zu bytes of 16-byte aligned workspace needed", need);
+  uint8_t* xq = static_cast<uint8_t*>(workspace);
+  float* xs = reinterpret_cast<float*>(xq + ((M * K + 15) & ~15LL));
+  const int rc = miq_fp8_quantize_rows(x, x_dtype, M, K, ldx, xq, xs, stream);
+  return rc != MIQ_OK ? rc : miq_fp8_gemm(xq, xs, wq, w_scale, y, ldy, M, N, K, stream);
+}

@@ -175,3 +175,19 @@ def fp8_gemm(x_fp8, x_scale, w_fp8, w_scale):
     L.call("miq_fp8_gemm", L.ptr(xq), L.ptr(xs), L.ptr(wq), L.ptr(wsc), L.ptr(y), N, M, N, K,
            L.stream(x_fp8.device))
     return y
+
+
+def fp8_linear(x, w_fp8, w_scale):
+    """FP8WeightAct.linear on a native device (fp8.py:48-61) in one library call: the rows of
+    x quantized into a scratch buffer, then the GEMM. K must be a multiple of 128."""
+    L.require_device(x, w_fp8, w_scale)
+    x2 = _contig_rows(x)
+    M, K = x2.shape
+    N = w_fp8.shape[0]
+    wq = w_fp8.contiguous()
+    wsc = w_scale.reshape(-1).float().contiguous()
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    ws = torch.empty(L.load().miq_fp8_linear_workspace_bytes(M, K), dtype=torch.uint8, device=x.device)
+    L.call("miq_fp8_linear", L.ptr(x2), L.dtype_code(x2.dtype), x2.stride(0), L.ptr(wq), L.ptr(wsc), L.ptr(y), N,
+           M, N, K, L.ptr(ws), ws.numel(), L.stream(x.device))
+    return y.reshape(*x.shape[:-1], N)

@@ -51,3 +51,22 @@ def test_fp8_gemm_repeats_bit_for_bit():
     first = ops.fp8_gemm(*args)
     for _ in range(3):
         assert torch.equal(ops.fp8_gemm(*args), first)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape,N,K", [((1,), 64, 128), ((3, 7), 96, 640), ((2, 600), 192, 256)])
+def test_fp8_linear_in_one_call_equals_two(shape, N, K, dtype):
+    """miq_fp8_linear = miq_fp8_quantize_rows + miq_fp8_gemm, byte for byte, for contiguous,
+    row-strided and misaligned (last-dim offset) activations."""
+    from engine.quantization import get_method
+    from kernels import quant_ops as ops
+    print(f"[case] fp8 linear {shape} N={N} K={K} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(K + N)
+    w = {k: v.to(DEV) for k, v in O.fp8_quantize((torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16)).items()}
+    m = get_method("fp8", device=DEV)
+    wide = torch.randn(*shape, K + 9, generator=g).to(dtype).to(DEV)
+    for x in (wide[..., :K].contiguous(), wide[..., :K], wide[..., 3:3 + K]):
+        q, s = ops.fp8_quantize_rows(x.reshape(-1, K))
+        want = ops.fp8_gemm(q, s, w["qweight"], w["scale"]).to(dtype).reshape(*shape, N)
+        got = m.linear(x, **w)
+        assert got.dtype == dtype and got.shape == want.shape and torch.equal(got, want)
