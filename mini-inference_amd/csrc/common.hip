@@ -58,6 +58,10 @@ Tuning read_tuning() {
   const char* ml = getenv("MIQ_MOE_LDS_SCALES");
   t.moe_no_lds_scales = ml && atoi(ml) == 0;
   t.moe_align_scan = flag("MIQ_MOE_ALIGN_SCAN");
+  const char* mb = getenv("MIQ_MOE_BLOCK");
+  t.moe_block = mb ? atoi(mb) : -1;
+  const char* wb = getenv("MIQ_WO_BLOCK");
+  t.wo_block = wb ? atoi(wb) : -1;
   t.moe_align_launch = flag("MIQ_MOE_ALIGN_LAUNCH");
   return t;
 }

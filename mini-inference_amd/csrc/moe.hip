@@ -24,6 +24,7 @@
 
 #include <type_traits>
 
+#include "wo_block.h"
 #include "wo_core.h"
 
 namespace miq {
@@ -193,6 +194,161 @@ moe_align_chunks_kernel(const void* __restrict__ ids, int dtype, int num_pairs, 
     const int e = le[i];
     sorted_ids[offsets[e] + cc[(i >> 6) * E + e] + r] = i;
   }
+}
+
+// The grouping of the block GEMMs (wo_block.hip) in one workgroup: experts padded to kGroupRows
+// rows, and the list of row tiles (up to kMoeTileRows rows; an expert's rows spread evenly over
+// its tiles). Ranks inside an expert come from ballots as above, and are formed again when the
+// pairs are placed, so 16 bits per (chunk of 64 pairs, expert) are all the LDS it takes (64
+// experts: up to 65535 pairs). A wavefront requests the ids of kGroupAhead chunks at once, and
+// 1024 / E threads per expert share the prefix over the chunks: one latency each instead of one
+// per chunk. OLMoE, 8000 pairs, MI355X: 89.8 us (moe_align, one wavefront per expert walking
+// all the pairs) -> 16 us.
+constexpr int kGroupRows = 32, kGroupAhead = 8;
+
+__global__ void __launch_bounds__(1024)
+moe_group_kernel(const void* __restrict__ ids, int dtype, int num_pairs, int E, int segs, int32_t* __restrict__ sorted_ids,
+                 int32_t* __restrict__ rank, MoeTile* __restrict__ tiles, int32_t* __restrict__ num_tiles) {
+  extern __shared__ int sm[];
+  constexpr int kBlocks = kMoeTileRows / kGroupRows;  // 32-row blocks per tile at most
+  const int nch = (num_pairs + 63) / 64;
+  int* counts = sm;            // [E] pairs of the expert
+  int* offsets = sm + E;       // [E + 1] first padded row
+  int* toff = sm + 2 * E + 1;  // [E] first tile
+  int* part = sm + 3 * E + 1;  // [segs][E] pairs of the expert in a segment of the chunks
+  uint16_t* cc = reinterpret_cast<uint16_t*>(part + segs * E);  // [nch][E] pairs in the chunk, then those before it
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int nw = 1024 / 64;
+  const int nbits = 32 - __builtin_clz((unsigned)E);  // ids 0 .. E (E: out of range)
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  // this lane's pair of chunk c: expert (E: none) | rank in the chunk among its pairs << 16; the
+  // chunk's first pair of an expert also has the expert's pairs in the chunk << 22
+  auto key_of = [&](int id) -> uint32_t {
+    const int e = id < 0 || id >= E ? E : id;
+    uint64_t peers = ~0ull;
+    for (int b = 0; b < nbits; ++b) {
+      const bool bit = (e >> b) & 1;
+      const uint64_t m = __ballot(bit);
+      peers &= bit ? m : ~m;
+    }
+    const int r = __popcll(peers & below);
+    return (uint32_t)e | (uint32_t)r << 16 | (r == 0 ? (uint32_t)__popcll(peers) << 22 : 0u);
+  };
+  // f(chunk, key) for this wavefront's chunks; the first kGroupAhead keys stay in registers
+  // between the two passes (up to 16 x kGroupAhead chunks need no second forming)
+  uint32_t held[kGroupAhead];
+  auto each_chunk = [&](bool have, auto&& f) {
+    for (int c0 = wv; c0 < nch; c0 += nw * kGroupAhead) {
+      int id[kGroupAhead];
+      if (!have || c0 != wv)
+#pragma unroll
+        for (int q = 0; q < kGroupAhead; ++q) {
+          const int i = (c0 + q * nw) * 64 + lane;
+          id[q] = i < num_pairs ? load_id(ids, dtype, i) : E;
+        }
+#pragma unroll
+      for (int q = 0; q < kGroupAhead; ++q) {
+        const int c = c0 + q * nw;
+        if (c >= nch) break;  // uniform
+        const uint32_t key = have && c0 == wv ? held[q] : key_of(id[q]);
+        if (!have && c0 == wv) held[q] = key;
+        f(c, key);
+      }
+    }
+  };
+  for (int i = tid; i < nch * E; i += 1024) cc[i] = 0;
+  __syncthreads();
+  each_chunk(false, [&](int c, uint32_t key) {
+    const int e = key & 0xffff;
+    if (e < E && (key >> 22)) cc[c * E + e] = (uint16_t)(key >> 22);
+  });
+  __syncthreads();
+  // exclusive prefix over the chunks: sums of `segs` segments of chunks, then each segment from
+  // the sum of those before it
+  const int seg_len = (nch + segs - 1) / segs;
+  for (int i = tid; i < segs * E; i += 1024) {
+    const int sg = i / E, e = i - sg * E;
+    int sum = 0;
+    for (int c = sg * seg_len; c < min(nch, (sg + 1) * seg_len); ++c) sum += cc[c * E + e];
+    part[i] = sum;
+  }
+  __syncthreads();
+  for (int i = tid; i < segs * E; i += 1024) {
+    const int sg = i / E, e = i - sg * E;
+    int run = 0;
+    for (int q = 0; q < sg; ++q) run += part[q * E + e];
+    for (int c = sg * seg_len; c < min(nch, (sg + 1) * seg_len); ++c) {
+      const int n = cc[c * E + e];
+      cc[c * E + e] = (uint16_t)run;
+      run += n;
+    }
+    if (sg == segs - 1) counts[e] = run;
+  }
+  __syncthreads();
+  if (wv == 0) {  // exclusive scans of the padded rows and of the tiles, 64 experts per round
+    int rows = 0, nt = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, nb = e < E ? (counts[e] + kGroupRows - 1) / kGroupRows : 0, tl = (nb + kBlocks - 1) / kBlocks;
+      int ir = nb, it = tl;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int ur = __shfl_up(ir, o, 64), ut = __shfl_up(it, o, 64);
+        if (lane >= o) {
+          ir += ur;
+          it += ut;
+        }
+      }
+      if (e < E) {
+        offsets[e] = rows + (ir - nb) * kGroupRows;
+        toff[e] = nt + it - tl;
+      }
+      rows += __shfl(ir, 63, 64) * kGroupRows;
+      nt += __shfl(it, 63, 64);
+    }
+    if (lane == 0) {
+      offsets[E] = rows;
+      *num_tiles = nt;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < E; e += 1024) {  // nb blocks over tl tiles, sizes differing by at most one
+    const int nb = (offsets[e + 1] - offsets[e]) / kGroupRows, tl = (nb + kBlocks - 1) / kBlocks;
+    int b = 0;
+    for (int t = 0; t < tl; ++t) {
+      const int n = nb / tl + (t < nb % tl ? 1 : 0);
+      tiles[toff[e] + t] = MoeTile{e, offsets[e] + b * kGroupRows, n, 0};
+      b += n;
+    }
+  }
+  for (int i = tid; i < E * kGroupRows; i += 1024) {  // the rows past an expert's pairs
+    const int e = i / kGroupRows, row = offsets[e] + counts[e] + i % kGroupRows;
+    if (row < offsets[e + 1]) sorted_ids[row] = num_pairs;
+  }
+  each_chunk(true, [&](int c, uint32_t key) {
+    const int i = c * 64 + lane, e = key & 0xffff;
+    if (i >= num_pairs) return;
+    const int pos = e < E ? offsets[e] + cc[c * E + e] + (int)(key >> 16 & 63) : -1;
+    rank[i] = pos;
+    if (pos >= 0) sorted_ids[pos] = i;
+  });
+}
+
+// The expert of every pair (-1: none) from moe_align's layout with 16-row tiles, for layers that
+// are given that layout and take the block GEMMs: they group the pairs anew.
+__global__ void __launch_bounds__(1024)
+moe_pair_experts_kernel(const int32_t* __restrict__ sorted_ids, const int32_t* __restrict__ expert_ids,
+                        const int32_t* __restrict__ num_padded, int num_pairs, int32_t* __restrict__ ids) {
+  for (int i = threadIdx.x; i < num_pairs; i += 1024) ids[i] = -1;
+  __syncthreads();
+  const int used = *num_padded;
+  for (int r = threadIdx.x; r < used; r += 1024) {
+    const int pair = sorted_ids[r];
+    if (pair < num_pairs) ids[pair] = expert_ids[r / kTile];
+  }
+}
+
+int moe_group_segs(int64_t E) { return (int)std::max<int64_t>(1, std::min<int64_t>(16, 1024 / E)); }
+size_t moe_group_lds(int64_t pairs, int64_t E) {
+  return (size_t)((3 + moe_group_segs(E)) * E + 2) * 4 + (size_t)((pairs + 63) / 64 * E) * 2;
 }
 
 struct MoeParams {
@@ -1053,6 +1209,20 @@ void launch_experts(const MoeParams& p, bool hz, int sd, dim3 gu_grid, dim3 dn_g
 #undef MIQ_EXPERTS
 }
 
+// Whether a routed layer takes the block GEMMs: int8 experts with more than 16 pairs each on
+// average. The streaming kernels read an expert's weights once per 16 rows; the block GEMMs once
+// per 160, with every MFMA fragment used by up to 160 rows. OLMoE layer, MI355X, T = 64 / 128 /
+// 144 / 256 / 512 / 1000 / 2000: streaming 82 / 103 / 136 / 185 / 283 / 547 / 987 us, block 101 /
+// 111 / 107 / 115 / 135 / 172 / 311 us (the weights alone: 86 us at the copy rate).
+int64_t block_rows(int64_t pairs, int64_t E) { return pairs + std::min(E, pairs) * (kGroupRows - 1); }
+bool moe_block_ok(int kind, int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
+  const int64_t pairs = T * topk;
+  const int force = tuning().moe_block;
+  if (kind != KIND_INT8 || force == 0 || pairs >= 65536 || moe_group_lds(pairs, E) > (size_t)150 * 1024) return false;
+  if (!moe_block_fits(T, topk, E, H, I, block_rows(pairs, E))) return false;
+  return force == 1 || pairs > 16 * E;
+}
+
 size_t max_padded_rows(int64_t num_pairs, int64_t E) { return (size_t)(num_pairs + E * (kTile - 1)); }
 
 }  // namespace
@@ -1093,14 +1263,37 @@ size_t moe_base_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) 
   return align_up(max_padded_rows(T * topk, E) * (size_t)I * 2) + align_up((size_t)T * topk * H * 2) +
          align_up((size_t)T * topk * 4);
 }
+// The block GEMMs' workspace: hbuf [rows, I] bf16 | ypair [T * topk, H] bf16 | rank [T * topk] |
+// sorted_ids [rows] | tiles | experts of the pairs (layers given moe_align's layout) | number of
+// tiles, rows = block_rows
+size_t moe_block_tiles(int64_t pairs, int64_t E) { return (size_t)(pairs / kMoeTileRows + std::min(E, pairs)); }
+size_t moe_block_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
+  const int64_t pairs = T * topk, rows = block_rows(pairs, E);
+  return align_up((size_t)(rows * I * 2)) + align_up((size_t)(pairs * H * 2)) + align_up((size_t)(pairs * 4)) +
+         align_up((size_t)rows * 4) + align_up(moe_block_tiles(pairs, E) * sizeof(MoeTile)) +
+         align_up((size_t)(pairs * 4)) + 256;
+}
 }  // namespace
 
 extern "C" size_t miq_moe_workspace_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
   const size_t rows = max_padded_rows(T * topk, E);
-  return moe_base_bytes(T, topk, E, H, I) + align_up(rows * 4) + align_up((rows + kTile - 1) / kTile * 4) + 256;
+  const size_t bytes = moe_base_bytes(T, topk, E, H, I) + align_up(rows * 4) + align_up((rows + kTile - 1) / kTile * 4) + 256;
+  return moe_block_ok(KIND_INT8, T, topk, E, H, I) ? std::max(bytes, moe_block_bytes(T, topk, E, H, I)) : bytes;
 }
 
 namespace {
+int launch_combine(const uint16_t* ypair, const int32_t* rank, int64_t T, int64_t topk, int64_t H, uint16_t* out,
+                   hipStream_t st, const char* name) {
+  const dim3 cgrid((unsigned)((H / 4 + 255) / 256), (unsigned)T);
+  if (topk <= 8)
+    hipLaunchKernelGGL(moe_combine_kernel<8>, cgrid, dim3(256), 0, st, ypair, rank, (int)topk, (int)H, out);
+  else if (topk <= 16)
+    hipLaunchKernelGGL(moe_combine_kernel<16>, cgrid, dim3(256), 0, st, ypair, rank, (int)topk, (int)H, out);
+  else
+    hipLaunchKernelGGL(moe_combine_kernel<32>, cgrid, dim3(256), 0, st, ypair, rank, (int)topk, (int)H, out);
+  return check_launch(name);
+}
+
 // Argument checks, workspace layout and launches shared by the INT4 and INT8 entry points.
 int run_moe(int kind, const void* hidden, int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk,
             const uint8_t* gu_q, const void* gu_scale, const void* gu_zero, const uint8_t* dn_q,
@@ -1151,11 +1344,58 @@ int run_moe(int kind, const void* hidden, int64_t T, int64_t H, int64_t I, int64
   p.w_dtype = w_dtype;
   const size_t max_rows = max_padded_rows(T * topk, E);
   hipStream_t st = (hipStream_t)stream;
+  MIQ_REQUIRE(!topk_ids || idx_dtype == MIQ_INT32 || idx_dtype == MIQ_INT64, "%s: topk_ids must be int32 or int64", name);
+  if ((topk_ids || (sorted_ids && expert_ids && num_padded)) && moe_block_ok(kind, T, topk, E, H, I)) {
+    const int64_t pairs = T * topk, rows = block_rows(pairs, E);
+    char* at = static_cast<char*>(workspace);
+    auto take = [&](size_t bytes) {
+      char* q = at;
+      at += align_up(bytes);
+      return q;
+    };
+    MoeBlockArgs a{};
+    a.hbuf = reinterpret_cast<uint16_t*>(take((size_t)(rows * I * 2)));
+    a.ypair = reinterpret_cast<uint16_t*>(take((size_t)(pairs * H * 2)));
+    int32_t* rank = reinterpret_cast<int32_t*>(take((size_t)(pairs * 4)));
+    int32_t* sorted = reinterpret_cast<int32_t*>(take((size_t)rows * 4));
+    MoeTile* tiles = reinterpret_cast<MoeTile*>(take(moe_block_tiles(pairs, E) * sizeof(MoeTile)));
+    int32_t* pair_ids = reinterpret_cast<int32_t*>(take((size_t)(pairs * 4)));
+    int32_t* num_tiles = reinterpret_cast<int32_t*>(at);
+    if (!topk_ids) {
+      hipLaunchKernelGGL(moe_pair_experts_kernel, dim3(1), dim3(1024), 0, st, sorted_ids, expert_ids, num_padded,
+                         (int)pairs, pair_ids);
+      topk_ids = pair_ids;
+      idx_dtype = MIQ_INT32;
+    }
+    a.hidden = p.hidden;
+    a.T = (int)T;
+    a.H = (int)H;
+    a.I = (int)I;
+    a.E = (int)E;
+    a.topk = (int)topk;
+    a.gu_q = gu_q;
+    a.gu_s = gu_scale;
+    a.dn_q = dn_q;
+    a.dn_s = dn_scale;
+    a.sd = sz_dtype;
+    a.topk_w = topk_weights;
+    a.w_dtype = w_dtype;
+    a.tiles = tiles;
+    a.num_tiles = num_tiles;
+    a.sorted_ids = sorted;
+    a.max_rows = rows;
+    static std::once_flag lds_once;
+    std::call_once(lds_once, [] { allow_max_dynamic_lds(reinterpret_cast<const void*>(&moe_group_kernel)); });
+    hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), moe_group_lds(pairs, E), st, topk_ids, idx_dtype, (int)pairs,
+                       (int)E, moe_group_segs(E), sorted, rank, tiles, num_tiles);
+    const int rc = moe_block_launch(a, st, name);
+    if (rc) return rc;
+    return launch_combine(a.ypair, rank, T, topk, H, static_cast<uint16_t*>(out), st, name);
+  }
   if (topk_ids) {
     // routed: the expert GEMMs form moe_align's layout themselves where the pairs and
     // experts fit their LDS tables and the streaming kernels take the layer (int4: H a
     // multiple of 128 and I of 64); otherwise moe_align runs into the workspace's tail
-    MIQ_REQUIRE(idx_dtype == MIQ_INT32 || idx_dtype == MIQ_INT64, "%s: topk_ids must be int32 or int64", name);
     const bool stream_path = i8 || (H % 128 == 0 && I % 64 == 0 && !tuning().moe_tiled);
     if (stream_path && T * topk <= kRtPairs && E <= kRtExperts && !tuning().moe_align_launch) {
       p.topk_ids = topk_ids;
@@ -1201,14 +1441,7 @@ int run_moe(int kind, const void* hidden, int64_t T, int64_t H, int64_t I, int64
   }
   int rc = check_launch(name);
   if (rc) return rc;
-  const dim3 cgrid((unsigned)((H / 4 + 255) / 256), (unsigned)T);
-  if (topk <= 8)
-    hipLaunchKernelGGL(moe_combine_kernel<8>, cgrid, dim3(256), 0, st, p.ypair, p.rank, (int)topk, (int)H, p.out);
-  else if (topk <= 16)
-    hipLaunchKernelGGL(moe_combine_kernel<16>, cgrid, dim3(256), 0, st, p.ypair, p.rank, (int)topk, (int)H, p.out);
-  else
-    hipLaunchKernelGGL(moe_combine_kernel<32>, cgrid, dim3(256), 0, st, p.ypair, p.rank, (int)topk, (int)H, p.out);
-  return check_launch(name);
+  return launch_combine(p.ypair, p.rank, T, topk, H, p.out, st, name);
 }
 }  // namespace
 

@@ -36,6 +36,7 @@
 
 #include "miq_common.h"
 #include "wo_core.h"
+#include "wo_block.h"
 #include "wo_wide.h"
 
 namespace miq {
@@ -514,6 +515,8 @@ int wo_prefill_launch(int kind, const uint16_t* x, int64_t ldx, const uint8_t* w
                       const void* zero, int sd, int group_steps, int64_t ngroups, uint16_t* y, int64_t ldy, int64_t M,
                       int N, int K, void* workspace, size_t ws_bytes, size_t counter_bytes, hipStream_t st,
                       const char* name) {
+  if (kind == KIND_INT8 && wo_block_planned(M, N, K, ldx, wide_plan(M, N, K, ldw)))
+    return wo_block_launch(x, ldx, w, scale, sd, y, ldy, M, N, K, st, name);
   // the wide kernel where it is planned and its workspace fits (the no-allocation entry
   // point's scratch may not hold it: then the prefill kernel)
   if (workspace != nullptr && ws_bytes > counter_bytes) {

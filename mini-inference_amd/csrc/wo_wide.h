@@ -13,6 +13,7 @@ namespace miq {
 struct WidePlan {
   int mt = 0, S = 1, split_steps = 0;
   size_t pack_bytes = 0, part_bytes = 0;
+  double us = 0.0;  // modelled time of the main and reduce kernels
   size_t bytes() const { return pack_bytes + part_bytes; }
 };
 

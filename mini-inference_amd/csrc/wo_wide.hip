@@ -572,6 +572,7 @@ WidePlan wo_wide_plan(int64_t M, int64_t N, int64_t K, int64_t ldw) {
         best.pack_bytes = pack;
         best.part_bytes = part;
         best_t = t;
+        best.us = t;
       }
     }
   }
