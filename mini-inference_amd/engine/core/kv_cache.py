@@ -77,8 +77,9 @@ def kv_quant_write(cache, scale, slots, x):
     if x.stride(-1) != 1:
         x = x.contiguous()
     per_launch = 65535  # tokens one launch takes
+    whole = x.shape[0] <= per_launch
     for a in range(0, x.shape[0], per_launch):
-        xa, sa = x[a:a + per_launch], slots[a:a + per_launch]
+        xa, sa = (x, slots) if whole else (x[a:a + per_launch], slots[a:a + per_launch])
         L.call("miq_kv_quant_write", L.ptr(xa), L.dtype_code(xa.dtype), xa.shape[0], xa.shape[1], xa.shape[2],
                xa.stride(0), xa.stride(1), L.ptr(sa), L.ptr(cache), L.dtype_code(cache.dtype),
                cache.stride(0), cache.stride(1), L.ptr(scale), L.dtype_code(scale.dtype),

@@ -31,9 +31,10 @@ class _QuantTensors:
             self.register_buffer(prefix + key, tensors[key])
 
     def _tensors(self, prefix, index=None):
+        held = self._buffers  # (a module attribute lookup costs a Python call per tensor)
         out = {}
         for key in self._qkeys:
-            t = getattr(self, prefix + key)
+            t = held[prefix + key] if prefix + key in held else getattr(self, prefix + key)
             out[key] = t if index is None else t[index]
         return out
 

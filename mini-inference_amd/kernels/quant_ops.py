@@ -17,15 +17,22 @@ MAX_X_ELEMS = 1 << 31
 
 
 def _rows(t):
+    if t.dim() == 2:
+        return t.shape[0]
     return math.prod(t.shape[:-1]) if t.dim() > 1 else 1
 
 
 def _contig_rows(w):
     """View w [..., K] as [rows, K] with a row stride; copies only if the last dim is strided."""
-    w2 = w.reshape(-1, w.shape[-1])
+    w2 = w if w.dim() == 2 else w.reshape(-1, w.shape[-1])
     if w2.stride(-1) != 1:
         w2 = w2.contiguous()
     return w2
+
+
+def _like_rows(y, x):
+    """y [rows of x, N] in x's leading dimensions."""
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], y.shape[-1])
 
 
 # ---------------------------------------------------------------- int8 weight-only
@@ -67,12 +74,12 @@ def w8a16_linear(x, qweight, scale):
     ws = L.wo_workspace(x.device, nbytes)
     L.call("miq_w8a16_gemm", L.ptr(x2), x2.stride(0), L.ptr(q), L.ptr(s), L.dtype_code(s.dtype), L.ptr(y), N,
            M, N, K, L.ptr(ws), ws.numel(), L.stream(x.device))
-    return y.reshape(*x.shape[:-1], N)
+    return _like_rows(y, x)
 
 
 def w8a16_supported(x, qweight):
-    M = _rows(x)
-    return (x.dtype == torch.bfloat16 and M >= 1 and M * x.shape[-1] < MAX_X_ELEMS and x.shape[-1] % 128 == 0
+    M, K = _rows(x), x.shape[-1]
+    return (x.dtype == torch.bfloat16 and M >= 1 and M * K < MAX_X_ELEMS and K % 128 == 0
             and qweight.shape[-2] % 16 == 0 and qweight.dim() == 2)
 
 
@@ -123,16 +130,14 @@ def w4a16_linear(x, qweight, scale, zero):
     ws = L.wo_workspace(x.device, nbytes)
     L.call("miq_w4a16_gemm", L.ptr(x2), x2.stride(0), L.ptr(q), L.ptr(s), L.ptr(z), L.dtype_code(s.dtype), group,
            L.ptr(y), N, M, N, K, L.ptr(ws), ws.numel(), L.stream(x.device))
-    return y.reshape(*x.shape[:-1], N)
+    return _like_rows(y, x)
 
 
 def w4a16_supported(x, qweight, scale):
-    M = _rows(x)
-    K = x.shape[-1]
-    if scale.shape[-1] == 0 or K % scale.shape[-1]:
+    M, K, groups = _rows(x), x.shape[-1], scale.shape[-1]
+    if groups == 0 or K % groups:
         return False
-    group = K // scale.shape[-1]
-    return (x.dtype == torch.bfloat16 and M >= 1 and M * K < MAX_X_ELEMS and group % 128 == 0
+    return (x.dtype == torch.bfloat16 and M >= 1 and M * K < MAX_X_ELEMS and K // groups % 128 == 0
             and qweight.shape[-2] % 16 == 0 and qweight.dim() == 2)
 
 
@@ -190,4 +195,4 @@ def fp8_linear(x, w_fp8, w_scale):
     ws = torch.empty(L.load().miq_fp8_linear_workspace_bytes(M, K), dtype=torch.uint8, device=x.device)
     L.call("miq_fp8_linear", L.ptr(x2), L.dtype_code(x2.dtype), x2.stride(0), L.ptr(wq), L.ptr(wsc), L.ptr(y), N,
            M, N, K, L.ptr(ws), ws.numel(), L.stream(x.device))
-    return y.reshape(*x.shape[:-1], N)
+    return _like_rows(y, x)
