@@ -18,6 +18,7 @@ runner read. Prefix caching and the admission watermark belong to the reference'
 scheduler and are not rebuilt: `register` is a no-op and `admit` reports 0 cached tokens.
 """
 import bisect
+from array import array
 from collections import deque
 from typing import NamedTuple
 
@@ -142,6 +143,10 @@ class PagedAllocator:
         blocks = torch.tensor(self.tables[req.id], dtype=torch.long)
         return blocks[pos // self.block_size] * self.block_size + pos % self.block_size
 
+    def slot(self, req, pos):
+        """The slot of one position, without tensors."""
+        return self.tables[req.id][pos // self.block_size] * self.block_size + pos % self.block_size
+
     def stored_tokens(self):
         return sum(self.length.values())
 
@@ -203,6 +208,10 @@ class ContiguousAllocator:
         base = self.ranges[req.id][0]
         return torch.arange(base + start, base + end)
 
+    def slot(self, req, pos):
+        """The slot of one position, without tensors."""
+        return self.ranges[req.id][0] + pos
+
     def stored_tokens(self):
         return sum(self.length.values())
 
@@ -226,12 +235,19 @@ def make_allocator(mode, capacity_tokens, block_size=16):
 def pack_block_tables(tables, lens, device):
     """Per-request page lists and context lengths -> (block_table int32 [B, width], zero
     padded, seq_lens int32 [B]) on `device`, the paged-attention kernel's operands."""
+    flat, width = flat_block_tables(tables)
+    table = torch.frombuffer(flat, dtype=torch.int32).view(len(tables), width)
+    return table.to(device, copy=True), torch.tensor(list(lens), dtype=torch.int32).to(device)
+
+
+def flat_block_tables(tables):
+    """The rows of a block table, zero padded to a common width (at least 1), as one C int array
+    (a tensor operation per row costs more than the whole table), and the width."""
     width = max(1, max(len(t) for t in tables))
-    table = torch.zeros(len(tables), width, dtype=torch.int32)
+    flat = array("i", bytes(4 * width * len(tables)))
     for row, ids in enumerate(tables):
-        if ids:
-            table[row, : len(ids)] = torch.as_tensor(ids, dtype=torch.int32)
-    return table.to(device), torch.tensor(list(lens), dtype=torch.int32).to(device)
+        flat[row * width:row * width + len(ids)] = array("i", ids)
+    return flat, width
 
 
 class CacheBookkeeping:
@@ -259,24 +275,28 @@ class CacheBookkeeping:
     def slots(self, req, start, end):
         return self.allocator.slots(req, start, end)
 
+    def slot(self, req, pos):
+        return self.allocator.slot(req, pos)
+
     def decode_tables(self, entries, device):
         """Page tables for the paged decode-attention kernel (reference kv_cache.py:403-420).
         entries: (request, context_length) pairs. Returns (block_table int32 [B, pages],
         seq_lens int32 [B], page_size, max_len). A paged cache hands over each request's
         block table cut to its context (page = block size); a contiguous one describes its
         range token by token (page = 1)."""
+        tables, lens, page = self.page_lists(entries)
+        table, seq_lens = pack_block_tables(tables, lens, device)
+        return table, seq_lens, page, max(lens)
+
+    def page_lists(self, entries):
+        """decode_tables on the host: (page ids per request, context lengths, page size)."""
         lens = [n for _, n in entries]
         if self.mode == "paged":
             a = self.allocator
-            tables = [a.tables[r.id][: a.blocks_for(n)] for r, n in entries]
-            page = a.block_size
-        else:
-            span = max(lens)
-            tables = [list(range(self.allocator.ranges[r.id][0], self.allocator.ranges[r.id][0] + span))
-                      for r, _ in entries]
-            page = 1
-        table, seq_lens = pack_block_tables(tables, lens, device)
-        return table, seq_lens, page, max(lens)
+            return [a.tables[r.id][: a.blocks_for(n)] for r, n in entries], lens, a.block_size
+        span = max(lens)
+        return [range(self.allocator.ranges[r.id][0], self.allocator.ranges[r.id][0] + span) for r, _ in entries], lens, 1
+
 
 class KVCache(CacheBookkeeping):
     """KV storage for all layers with its allocator (reference kv_cache.py:305-425).

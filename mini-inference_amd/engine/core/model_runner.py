@@ -31,9 +31,12 @@ The reference's scheduler, CUDA-graph capture and fused projections are serving-
 features outside this path; `generate` below runs a fixed set of prompts greedily.
 """
 import itertools
+from array import array
 
 import torch
 import torch.nn.functional as F
+
+from engine.core.kv_cache import CacheBookkeeping, flat_block_tables
 
 SUPPORTED = ("OlmoeForCausalLM", "Qwen3ForCausalLM", "Qwen3MoeForCausalLM", "Qwen2ForCausalLM")
 _PAGED_BACKENDS = ("triton", "paged")
@@ -82,6 +85,11 @@ class Request:
     def all_ids(self):
         return self.prompt_ids + self.output_ids
 
+    def ids(self, start, end):
+        """all_ids[start:end] (0 <= start <= end) without joining the lists."""
+        n = len(self.prompt_ids)
+        return self.prompt_ids[start:end] + self.output_ids[max(start - n, 0):max(end - n, 0)]
+
     @property
     def total_len(self):
         return len(self.prompt_ids) + len(self.output_ids)
@@ -110,23 +118,47 @@ class BatchMetadata:
         firsts = [e - n for e, n in zip(ends, lengths)]  # first row of each chunk
         is_decode = [n == 1 and start > 0 for n, (_, start, _) in zip(lengths, chunks)]
 
-        token_ids = [t for req, start, end in chunks for t in req.all_ids[start:end]]
+        # this library's own cache hands out slots and pages as plain integers; another one is asked
+        # through its slots() and decode_tables()
+        own = (isinstance(cache, CacheBookkeeping) and type(cache).slots is CacheBookkeeping.slots
+               and type(cache).decode_tables is CacheBookkeeping.decode_tables)
+        token_ids, positions, slots = [], [], []
+        for n, (req, start, end) in zip(lengths, chunks):
+            token_ids += req.ids(start, end) if type(req) is Request else req.all_ids[start:end]
+            positions += range(start, end)
+            slots += [cache.slot(req, start)] if n == 1 and own else cache.slots(req, start, end).tolist()
         self.num_tokens = ends[-1] if ends else 0
-        self.input_ids = torch.tensor(token_ids, dtype=torch.long, device=device)
-        self.positions = torch.cat([torch.arange(s, e) for _, s, e in chunks]).to(device)
-        self.write_slots = torch.cat([cache.slots(r, s, e) for r, s, e in chunks]).to(device)
-        self.last_rows = torch.tensor([e - 1 for e in ends], dtype=torch.long, device=device)
         self.context_tokens = sum(end for _, _, end in chunks)
 
         self.prefill = [(first, end - start, start, cache.slots(req, 0, end).to(device))
                         for first, dec, (req, start, end) in zip(firsts, is_decode, chunks) if not dec]
         decodes = [(first, req, end) for first, dec, (req, _, end) in zip(firsts, is_decode, chunks) if dec]
-        self.decode_rows = torch.tensor([row for row, _, _ in decodes], dtype=torch.long, device=device)
         self.all_decode = not self.prefill
         self.decode_tables = None
-        if decodes and attn_backend in _PAGED_BACKENDS:
-            tables = cache.decode_tables([(req, end) for _, req, end in decodes], device)
-            self.decode_tables = (*tables, None)
+        paged = decodes and attn_backend in _PAGED_BACKENDS
+        entries = [(req, end) for _, req, end in decodes]
+        tables, lens, page = cache.page_lists(entries) if paged and own else ((), (), 0)
+        flat, width = flat_block_tables(tables) if paged and own else (array("i"), 0)
+        # one host buffer and one copy for everything the step indexes by: five int64 lists, then
+        # the block table and the context lengths as int32 (a copy per list costs a launch and a
+        # wait each)
+        parts = [token_ids, positions, slots, [e - 1 for e in ends], [row for row, _, _ in decodes]]
+        ints = array("q", itertools.chain.from_iterable(parts))
+        flat.extend(lens)
+        if len(flat) % 2:
+            flat.append(0)
+        ints.frombytes(flat.tobytes())
+        held = torch.frombuffer(ints, dtype=torch.int64).to(device, copy=True) if ints else torch.empty(
+            0, dtype=torch.int64, device=device)
+        at = list(itertools.accumulate((len(p) for p in parts), initial=0))
+        self.input_ids, self.positions, self.write_slots, self.last_rows, self.decode_rows = (
+            held[a:b] for a, b in zip(at, at[1:]))
+        if paged and not own:
+            self.decode_tables = (*cache.decode_tables(entries, device), None)
+        elif paged:
+            words = held[at[-1]:].view(torch.int32)
+            n = len(lens)
+            self.decode_tables = (words[:n * width].view(n, width), words[n * width:n * width + n], page, max(lens), None)
         elif decodes:
             slots = [cache.slots(req, 0, end) for _, req, end in decodes]
             width = max(len(s) for s in slots)
