@@ -192,6 +192,20 @@ int miq_kv_quant_write(const void* x, int x_dtype, int64_t T, int64_t heads, int
                        void* cache_scale, int scale_dtype, int64_t s_stride_t,
                        int64_t s_stride_h, void* stream);
 
+/* RoPE and the KV write of one layer's step in one launch: replaces the runner's
+ *   q = q * cos + rotate_half(q) * sin,  k likewise  (engine/core/model_runner.py:139-195)
+ * with its bf16 rounding after each product and sum, then KVCache.write of k and v
+ * (kv_cache.py:359-388, as miq_kv_quant_write). q: bf16 [T, heads, D], k, v: bf16 [T, kv_heads,
+ * D] (strides in elements), cos, sin: bf16 [T, D] (row stride cs_stride_t), D == 128; q_out: bf16
+ * [T, heads, D] contiguous; k_cache and v_cache (and k_scale and v_scale) share strides. */
+int miq_rope_kv_write(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k,
+                      int64_t k_stride_t, int64_t k_stride_h, const void* v, int64_t v_stride_t,
+                      int64_t v_stride_h, const void* cos, const void* sin, int64_t cs_stride_t,
+                      int64_t T, int64_t heads, int64_t kv_heads, int64_t D, const int64_t* slots,
+                      void* q_out, void* k_cache, void* v_cache, int kv_dtype, int64_t c_stride_t,
+                      int64_t c_stride_h, void* k_scale, void* v_scale, int scale_dtype,
+                      int64_t s_stride_t, int64_t s_stride_h, void* stream);
+
 /* ------------------------------------------------------------------ paged decode attention
  * Replaces paged_decode_attention (kernels/paged_attention/decode_triton.py:123-180):
  *   out[b, h] = softmax(sm_scale * q[b,h] . K_b^T) V_b over seq_lens[b] tokens, token i

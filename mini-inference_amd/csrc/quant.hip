@@ -231,6 +231,11 @@ __global__ void fp8_dequantize_kernel(const uint8_t* __restrict__ q, const float
 
 // ---------------------------------------------------------------- KV quantize-on-write
 // (kv_cache.py:359-388). One wavefront per (token, head).
+__device__ inline uint8_t kv_code(float v, bool is_int8) {
+  if (is_int8) return static_cast<uint8_t>(static_cast<int8_t>(fminf(fmaxf(__builtin_rintf(v), -127.f), 127.f)));
+  return f32_to_fp8(fminf(fmaxf(v, -448.f), 448.f));
+}
+
 __global__ void __launch_bounds__(64)
 kv_quant_write_kernel(const void* __restrict__ x, int x_dtype, int64_t heads, int64_t D,
                       int64_t xs_t, int64_t xs_h, const int64_t* __restrict__ slots,
@@ -248,15 +253,65 @@ kv_quant_write_kernel(const void* __restrict__ x, int x_dtype, int64_t heads, in
   const int64_t slot = slots[t];
   uint8_t* dst = cache + slot * cs_t + h * cs_h;
   for (int64_t d = threadIdx.x; d < D; d += 64) {
-    const float v = load_scalar(x, x_dtype, xb + d) / s;
-    if (is_int8) {
-      const float r = fminf(fmaxf(__builtin_rintf(v), -127.f), 127.f);
-      dst[d] = static_cast<uint8_t>(static_cast<int8_t>(r));
-    } else {
-      dst[d] = f32_to_fp8(fminf(fmaxf(v, -448.f), 448.f));
-    }
+    dst[d] = kv_code(load_scalar(x, x_dtype, xb + d) / s, is_int8);
   }
   if (threadIdx.x == 0) store_scalar(cscale, scale_dtype, slot * ss_t + h * ss_h, s);
+}
+
+// RoPE and the KV write of one layer in one launch: q and k rotated as torch does it in bf16 (each
+// product and the sum rounded), q to q_out, k and v quantized into the caches as
+// kv_quant_write_kernel does. One wavefront per (token, head) of q, k and v; lane l holds
+// elements l and l + 64 of the 128, which is the pair that the rotation mixes. In place of
+// twelve elementwise torch launches and two KV writes of 3-6 us each per layer, latency-bound
+// all of them at decode sizes (16 tokens, 32 + 8 + 8 heads: 14 launches, about 56 us on the GPU
+// -> one of 3.7 us).
+struct RopeKvParams {
+  const uint16_t *q, *k, *v, *cos, *sin;
+  int64_t q_t, q_h, k_t, k_h, v_t, v_h, cs_t;  // strides in elements
+  int heads, kv_heads;
+  const int64_t* slots;
+  uint16_t* q_out;                             // [T, heads, 128]
+  uint8_t *kc, *vc;
+  int kv_dtype;
+  int64_t c_t, c_h;
+  void *ks, *vs;
+  int scale_dtype;
+  int64_t s_t, s_h;
+};
+
+__global__ void __launch_bounds__(256) rope_kv_write_kernel(RopeKvParams p) {
+  const int lane = threadIdx.x & 63;
+  const int64_t t = blockIdx.y;
+  int h = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (h >= p.heads + 2 * p.kv_heads) return;  // whole wavefronts
+  const int kind = h < p.heads ? 0 : h < p.heads + p.kv_heads ? 1 : 2;  // q, k, v
+  h -= kind == 0 ? 0 : kind == 1 ? p.heads : p.heads + p.kv_heads;
+  const uint16_t* src = kind == 0 ? p.q + t * p.q_t + h * p.q_h
+                        : kind == 1 ? p.k + t * p.k_t + h * p.k_h : p.v + t * p.v_t + h * p.v_h;
+  float lo = bf16_to_f32(src[lane]), hi = bf16_to_f32(src[lane + 64]);
+  if (kind != 2) {
+    const uint16_t *c = p.cos + t * p.cs_t, *s = p.sin + t * p.cs_t;
+    auto mul = [](float a, uint16_t b) { return bf16_to_f32(f32_to_bf16(a * bf16_to_f32(b))); };
+    const float nlo = mul(lo, c[lane]) + mul(-hi, s[lane]);
+    const float nhi = mul(hi, c[lane + 64]) + mul(lo, s[lane + 64]);
+    const uint16_t blo = f32_to_bf16(nlo), bhi = f32_to_bf16(nhi);
+    if (kind == 0) {
+      uint16_t* dst = p.q_out + (t * p.heads + h) * 128;
+      dst[lane] = blo;
+      dst[lane + 64] = bhi;
+      return;
+    }
+    lo = bf16_to_f32(blo);
+    hi = bf16_to_f32(bhi);
+  }
+  const bool is_int8 = p.kv_dtype == MIQ_INT8;
+  const float amax = wave_max(fmaxf(fmaxf(0.f, fabsf(lo)), fabsf(hi)));
+  const float s = round_to(fmaxf(amax / (is_int8 ? 127.0f : 448.0f), 1e-8f), p.scale_dtype);
+  const int64_t slot = p.slots[t];
+  uint8_t* dst = (kind == 1 ? p.kc : p.vc) + slot * p.c_t + h * p.c_h;
+  dst[lane] = kv_code(lo / s, is_int8);
+  dst[lane + 64] = kv_code(hi / s, is_int8);
+  if (lane == 0) store_scalar(kind == 1 ? p.ks : p.vs, p.scale_dtype, slot * p.s_t + h * p.s_h, s);
 }
 
 inline bool is_float_dtype(int d) { return d == MIQ_F32 || d == MIQ_BF16 || d == MIQ_F16; }
@@ -373,4 +428,50 @@ extern "C" int miq_kv_quant_write(const void* x, int x_dtype, int64_t T, int64_t
                      static_cast<uint8_t*>(cache), kv_dtype, c_stride_t, c_stride_h, cache_scale,
                      scale_dtype, s_stride_t, s_stride_h);
   return check_launch("kv_quant_write");
+}
+
+extern "C" int miq_rope_kv_write(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k,
+                                 int64_t k_stride_t, int64_t k_stride_h, const void* v, int64_t v_stride_t,
+                                 int64_t v_stride_h, const void* cos, const void* sin, int64_t cs_stride_t, int64_t T,
+                                 int64_t heads, int64_t kv_heads, int64_t D, const int64_t* slots, void* q_out,
+                                 void* k_cache, void* v_cache, int kv_dtype, int64_t c_stride_t, int64_t c_stride_h,
+                                 void* k_scale, void* v_scale, int scale_dtype, int64_t s_stride_t,
+                                 int64_t s_stride_h, void* stream) {
+  MIQ_REQUIRE(is_float_dtype(scale_dtype), "rope_kv_write: bad scale dtype");
+  MIQ_REQUIRE(kv_dtype == MIQ_INT8 || kv_dtype == MIQ_FP8_E4M3, "rope_kv_write: kv_dtype must be int8 or fp8");
+  MIQ_REQUIRE(D == 128, "rope_kv_write: D=%lld must be 128", (long long)D);
+  MIQ_REQUIRE(T >= 0 && T < 65536 && heads > 0 && kv_heads > 0 && heads < 65536 && kv_heads < 65536,
+              "rope_kv_write: bad shape T=%lld heads=%lld kv_heads=%lld", (long long)T, (long long)heads,
+              (long long)kv_heads);
+  if (T == 0) return MIQ_OK;
+  RopeKvParams p{};
+  p.q = static_cast<const uint16_t*>(q);
+  p.k = static_cast<const uint16_t*>(k);
+  p.v = static_cast<const uint16_t*>(v);
+  p.cos = static_cast<const uint16_t*>(cos);
+  p.sin = static_cast<const uint16_t*>(sin);
+  p.q_t = q_stride_t;
+  p.q_h = q_stride_h;
+  p.k_t = k_stride_t;
+  p.k_h = k_stride_h;
+  p.v_t = v_stride_t;
+  p.v_h = v_stride_h;
+  p.cs_t = cs_stride_t;
+  p.heads = (int)heads;
+  p.kv_heads = (int)kv_heads;
+  p.slots = slots;
+  p.q_out = static_cast<uint16_t*>(q_out);
+  p.kc = static_cast<uint8_t*>(k_cache);
+  p.vc = static_cast<uint8_t*>(v_cache);
+  p.kv_dtype = kv_dtype;
+  p.c_t = c_stride_t;
+  p.c_h = c_stride_h;
+  p.ks = k_scale;
+  p.vs = v_scale;
+  p.scale_dtype = scale_dtype;
+  p.s_t = s_stride_t;
+  p.s_h = s_stride_h;
+  const unsigned gx = (unsigned)((heads + 2 * kv_heads + 3) / 4);
+  hipLaunchKernelGGL(rope_kv_write_kernel, dim3(gx, (unsigned)T), dim3(256), 0, (hipStream_t)stream, p);
+  return check_launch("rope_kv_write");
 }

@@ -87,6 +87,26 @@ def kv_quant_write(cache, scale, slots, x):
                scale.stride(0), scale.stride(1), L.stream(x.device))
 
 
+def rotate_half(x):
+    lo, hi = x.chunk(2, dim=-1)
+    return torch.cat((-hi, lo), dim=-1)
+
+
+def rope_kv_write(k_cache, v_cache, k_scale, v_scale, slots, q, k, v, cos, sin):
+    """KVCache.write_rotated's kernel on one layer's caches; returns the rotated q."""
+    L.require_device(q, k, v, cos, sin, slots, k_cache)
+    T, heads, D = q.shape
+    if slots.dtype != torch.int64 or not slots.is_contiguous():
+        slots = slots.to(torch.int64).contiguous()
+    out = torch.empty((T, heads, D), dtype=torch.bfloat16, device=q.device)
+    L.call("miq_rope_kv_write", L.ptr(q), q.stride(0), q.stride(1), L.ptr(k), k.stride(0), k.stride(1),
+           L.ptr(v), v.stride(0), v.stride(1), L.ptr(cos), L.ptr(sin), cos.stride(0), T, heads, k.shape[1], D,
+           L.ptr(slots), L.ptr(out), L.ptr(k_cache), L.ptr(v_cache), L.dtype_code(k_cache.dtype),
+           k_cache.stride(0), k_cache.stride(1), L.ptr(k_scale), L.ptr(v_scale), L.dtype_code(k_scale.dtype),
+           k_scale.stride(0), k_scale.stride(1), L.stream(q.device))
+    return out
+
+
 def _cdiv(a, b):
     return -(-a // b)
 
@@ -332,6 +352,24 @@ class KVCache(CacheBookkeeping):
         slots = slots.to(torch.int64).contiguous()
         kv_quant_write(self.k[layer], self.k_scale[layer], slots, k)
         kv_quant_write(self.v[layer], self.v_scale[layer], slots, v)
+
+    def write_rotated(self, layer, slots, q, k, v, cos, sin):
+        """RoPE of q and k and the write of k and v: returns q rotated. q [T, heads, D], k and v
+        [T, kv_heads, D], cos and sin [T, 1, D]. bf16 steps into an 8-bit cache on the device take
+        one kernel (rope_kv_write, the same roundings); the rest the formula itself."""
+        if (self.kv_dtype is not None and q.is_cuda and type(self).write is KVCache.write and 0 < q.shape[0] < 65536
+                and q.shape[-1] == 128 and all(t.dtype == torch.bfloat16 for t in (q, k, v, cos, sin))
+                and all(t.stride(-1) == 1 for t in (q, k, v)) and cos.stride() == sin.stride()
+                and cos.shape == sin.shape == (q.shape[0], 1, 128) and cos.stride(-1) == 1
+                and k.shape == v.shape == (q.shape[0], self.k.shape[2], 128) and slots.numel() == q.shape[0]
+                and self.k.stride() == self.v.stride()
+                and self.k_scale.stride() == self.v_scale.stride()):
+            return rope_kv_write(self.k[layer], self.v[layer], self.k_scale[layer], self.v_scale[layer], slots, q, k, v,
+                                 cos, sin)
+        q = q * cos + rotate_half(q) * sin
+        k = k * cos + rotate_half(k) * sin
+        self.write(layer, slots, k, v)
+        return q
 
     def _codes(self, t, layer, idx):
         if t.dtype == torch.float8_e4m3fn:  # advanced indexing of fp8 goes through the raw bytes

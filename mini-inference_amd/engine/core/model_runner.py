@@ -36,15 +36,10 @@ from array import array
 import torch
 import torch.nn.functional as F
 
-from engine.core.kv_cache import CacheBookkeeping, flat_block_tables
+from engine.core.kv_cache import CacheBookkeeping, flat_block_tables, rotate_half
 
 SUPPORTED = ("OlmoeForCausalLM", "Qwen3ForCausalLM", "Qwen3MoeForCausalLM", "Qwen2ForCausalLM")
 _PAGED_BACKENDS = ("triton", "paged")
-
-
-def rotate_half(x):
-    lo, hi = x.chunk(2, dim=-1)
-    return torch.cat((-hi, lo), dim=-1)
 
 
 def describe(model):
@@ -227,9 +222,13 @@ class ModelRunner:
 
     def _attention(self, layer_idx, attn, h, cos, sin, meta):
         q, k, v = self._project(attn, h, meta.num_tokens)
-        q = q * cos + rotate_half(q) * sin
-        k = k * cos + rotate_half(k) * sin
-        self.cache.write(layer_idx, meta.write_slots, k, v)
+        write_rotated = getattr(self.cache, "write_rotated", None)
+        if write_rotated is not None:
+            q = write_rotated(layer_idx, meta.write_slots, q, k, v, cos, sin)
+        else:  # a cache of another library
+            q = q * cos + rotate_half(q) * sin
+            k = k * cos + rotate_half(k) * sin
+            self.cache.write(layer_idx, meta.write_slots, k, v)
 
         if meta.all_decode and meta.decode_tables is not None:
             out = self._paged_decode(layer_idx, attn, q, meta)

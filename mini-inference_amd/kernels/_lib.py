@@ -54,6 +54,8 @@ SIGNATURES = {
     "miq_fp8_linear": (_I32, [_P, _I32, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _SZ, _P]),
     "miq_kv_quant_write": (_I32, [_P, _I32, _I64, _I64, _I64, _I64, _I64, _P, _P, _I32, _I64, _I64,
                                   _P, _I32, _I64, _I64, _P]),
+    "miq_rope_kv_write": (_I32, [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64,
+                                 _P, _P, _P, _P, _I32, _I64, _I64, _P, _P, _I32, _I64, _I64, _P]),
     "miq_paged_decode": (_I32, [_P, _I64, _I64, _P, _P, _I32, _I64, _I64, _P, _P, _I32, _I64, _I64,
                                 _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _F32, _I64, _I64, _P, _P,
                                 _P, _I64, _I64, _P]),
