@@ -145,14 +145,21 @@ __device__ inline void block(const BlockParams& p, uint8_t* smem, int m0, int nb
     woff[u] = n >= 0 ? n * p.K + (((lane & 3) ^ ((row >> 2) & 3)) << 4) : kOutB;
     wdst[u] = kXBytes<WM> + b * 1024;
   }
-  auto issue = [&](int s, int slot) {
+  // this wavefront's loads u = part, part + parts, ... of stage s into ring slot `slot` (zeros, and
+  // no memory traffic, past the last stage: every stage has the same loads in flight)
+  const int nst = p.K / kBK;
+  auto issue = [&](int s, int slot, int part, int parts) {
     uint8_t* base = smem + slot * kStageBytes<WM>;
+    const uint32_t kx = s < nst ? (uint32_t)s * (kBK * 2) : (uint32_t)kOutB, kw = s < nst ? (uint32_t)s * kBK : (uint32_t)kOutB;
 #pragma unroll
-    for (int u = 0; u < nX; ++u)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_ptr)(base + xdst[u]), 16, xoff[u] + s * (kBK * 2), 0, 0, 0);
-#pragma unroll
-    for (int u = 0; u < nW; ++u)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_ptr)(base + wdst[u]), 16, woff[u] + s * kBK, 0, 0, 0);
+    for (int u = 0; u < nX + nW; ++u) {
+      if (u % parts != part) continue;
+      if (u < nX)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_ptr)(base + xdst[u]), 16, (int)((uint32_t)xoff[u] + kx), 0, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_ptr)(base + wdst[u - nX]), 16,
+                                                 (int)((uint32_t)woff[u - nX] + kw), 0, 0, 0);
+    }
   };
 
   f32x16 acc[MT][2];
@@ -207,18 +214,17 @@ __device__ inline void block(const BlockParams& p, uint8_t* smem, int m0, int nb
       __builtin_amdgcn_sched_group_barrier(0x2, 24 / (2 * MT), 0);  // VALU
     }
   };
-  const int nst = p.K / kBK;
-  issue(0, 0);
-  issue(1, 1);  // K is a multiple of 128: at least two stages
+  issue(0, 0, 0, 1);
+  issue(1, 1, 0, 1);
   int slot = 0, free_slot = 2;
   for (int s = 0; s < nst; ++s) {
     // this wavefront's loads of stage s have landed (those of stage s + 1 may be in flight);
-    // after the barrier everyone's have, and stage s - 1's slot is free
-    if (s + 1 < nst) wait_loads<nX + nW>();
-    else wait_loads<0>();
+    // after the barrier everyone's have, and stage s - 1's slot is free. The next loads go out
+    // a few at a time between the sub-steps: all at once they filled the address units' queue
+    // and the wavefront's MFMAs waited behind them.
+    wait_loads<nX + nW>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (s + 2 < nst) issue(s + 2, free_slot);
-    const int base = slot * kStageBytes<WM>;
+    const int base = slot * kStageBytes<WM>, fill = free_slot;
     slot = slot == kStages - 1 ? 0 : slot + 1;
     free_slot = free_slot == kStages - 1 ? 0 : free_slot + 1;
     read_w(base, 0);
@@ -231,6 +237,7 @@ __device__ inline void block(const BlockParams& p, uint8_t* smem, int m0, int nb
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       read_x(base, c + 1);
+      issue(s + 2, fill, c, 3);
       __builtin_amdgcn_sched_barrier(0);
       multiply(c);
       convert(c + 1);
