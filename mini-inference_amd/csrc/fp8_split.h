@@ -6,9 +6,10 @@
 
 namespace miq {
 
-// 16 mt x 16 nt tiles, nw wavefronts per workgroup that split K (mt = 0: not this kernel).
+// 16 mt x 16 nt tiles, nw wavefronts per workgroup that split K, and the modelled time.
 struct Fp8SplitPlan {
   int mt = 0, nt = 0, nw = 0;
+  double us = 0.0;
 };
 
 Fp8SplitPlan fp8_split_plan(int64_t M, int64_t N, int64_t K);

@@ -167,8 +167,7 @@ void go(const SplitParams& p, hipStream_t st) {
 
 }  // namespace
 
-// Tile sizes and wavefronts of a call, or mt = 0 where the LDS-staged 128 x 128 tiles of
-// fp8_gemm.hip are expected to be faster. The kernel runs at the rate at which a CU pulls
+// Tile sizes, wavefronts and modelled time of a call. The kernel runs at the rate at which a CU pulls
 // operands from L2, so the plan takes the tile that needs the fewest bytes on the busiest CU
 // (tiles per CU, rounded up, times the tile's rows; activation rows, read 64 bytes at a time,
 // weigh 1.3 times the weights' whole lines), and fewer wavefronts per workgroup where a CU
@@ -176,9 +175,9 @@ void go(const SplitParams& p, hipStream_t st) {
 // K = 6144 x 2560, 2560 x 9728, 19456 x 2560, 2560 x 4096 and 1024 x 1024 at M = 1 .. 1000: the
 // plan is within 10 % of the fastest tile. Split against 128 x 128 tiles, us (rotating weight
 // copies): 6144 x 2560 M = 1 / 16 / 64 / 256 / 512: 6 / 7 / 11 / 21 / 31 against 31 / 33 / 40 /
-// 42 / 41; 2560 x 9728: 8 / 11 / 17 / 31 / 54 against 101 / 102 / 110 / 113 / 110. The line
-// between the two compares 4 us + bytes / 42 KB per us with 1.45 us per k-step and round of
-// 256 tiles (at 19456 x 2560 the two meet near M = 256: 49.6 against 48.5 us).
+// 42 / 41; 2560 x 9728: 8 / 11 / 17 / 31 / 54 against 101 / 102 / 110 / 113 / 110. Modelled
+// time (miq_fp8_gemm compares it with the other kernels'): 4 us, those bytes at 41 (K = 2560) to
+// 59 KB (K = 9728) per us, and 0.1 us per MB of weights.
 Fp8SplitPlan fp8_split_plan(int64_t M, int64_t N, int64_t K) {
   static const int kTiles[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {4, 2}, {4, 4}};
   Fp8SplitPlan best;
@@ -195,12 +194,11 @@ Fp8SplitPlan fp8_split_plan(int64_t M, int64_t N, int64_t K) {
   }
   const int64_t steps = K / kStep;
   while (best.nw > 2 && steps < 2 * best.nw) best.nw /= 2;
-  const double rounds = (double)(((M + 127) / 128) * ((N + 127) / 128)) / 256.0;
-  if (4.0 + best_bytes / 42e3 > 1.45 * (double)steps * std::max(1.0, rounds)) best.mt = 0;
+  best.us = 4.0 + best_bytes / (34e3 + 330.0 * (double)std::min<int64_t>(steps, 76)) + 1e-7 * (double)N * (double)K;
   return best;
 }
 
-// Launches the planned tile (pl.mt != 0); operands below 2 GiB, K a multiple of 128.
+// Launches the planned tile; operands below 2 GiB, K a multiple of 128.
 int fp8_split_launch(const Fp8SplitPlan& pl, const uint8_t* xq, const float* xs, const uint8_t* wq, const float* ws,
                      uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K, hipStream_t st) {
   SplitParams p{xq, xs, wq, ws, y, ldy, (int)M, (int)N, (int)K, 0, 0, false};
