@@ -62,6 +62,8 @@ Tuning read_tuning() {
   t.moe_block = mb ? atoi(mb) : -1;
   const char* wb = getenv("MIQ_WO_BLOCK");
   t.wo_block = wb ? atoi(wb) : -1;
+  const char* wsp = getenv("MIQ_WO_SPLIT");
+  t.wo_split = wsp ? atoi(wsp) : -1;
   t.moe_align_launch = flag("MIQ_MOE_ALIGN_LAUNCH");
   return t;
 }

@@ -216,6 +216,7 @@ struct Tuning {
   bool moe_align_scan;        // MIQ_MOE_ALIGN_SCAN: the one-wavefront-per-expert align
   int moe_block;              // MIQ_MOE_BLOCK: block expert GEMMs: 0 off, 1 wherever they apply, -1 default
   int wo_block;               // MIQ_WO_BLOCK: INT8 block GEMM (M > 64): 0 off, 1 wherever it applies, -1 default
+  int wo_split;               // MIQ_WO_SPLIT: INT8 split kernel: 0 off, 1 wherever it applies, -1 default
   bool moe_align_launch;      // MIQ_MOE_ALIGN_LAUNCH: routed MoE entry points run moe_align
 };
 const Tuning& tuning();

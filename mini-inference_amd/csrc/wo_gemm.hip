@@ -2,12 +2,15 @@
 //
 //   y[m, n] = sum_k x[m, k] * W[n, k],  x bf16 [M, K],  W int8 [N, K] or int4 [N, K/2]
 //
-// Argument checks live here. Up to 16 rows whose activations fit LDS run the one-tile-per-
-// workgroup kernel (wo_tile.hip); the rest the streamed split-K kernel (wo_stream.hip).
+// Argument checks live here. INT8 batches of 17 to 64 rows (5 to 16 where its tiles are small) run
+// the split kernel (wo_split.hip). Otherwise up to 16 rows whose activations fit LDS run the
+// one-tile-per-workgroup kernel (wo_tile.hip); the rest the streamed split-K kernel
+// (wo_stream.hip).
 #include <algorithm>
 #include <mutex>
 
 #include "wo_core.h"
+#include "wo_split.h"
 
 namespace miq {
 
@@ -62,6 +65,11 @@ int run(int kind, const WoArgs& p, void* workspace, size_t ws_bytes, hipStream_t
               "%s: x must be 16-byte aligned with a row stride multiple of 8", name);
   MIQ_REQUIRE((reinterpret_cast<uintptr_t>(p.w) & 15) == 0, "%s: weights must be 16-byte aligned", name);
   MIQ_REQUIRE(p.ldx >= p.K && p.ldy >= p.N, "%s: bad strides", name);
+  if (kind == KIND_INT8) {  // decode batches (and some short prefills): the split kernel
+    const WoSplitPlan pl = wo_split_plan(p.M, p.N, p.K, p.ldx);
+    if (pl.mt != 0)
+      return wo_split_launch(pl, p.x, p.ldx, p.w, p.scale, p.sz_dtype, p.y, p.ldy, p.M, p.N, p.K, st, name);
+  }
   if (p.M >= tuning().wo_prefill_min_m)  // prefill (M > 64): the dequantize-in-the-K-loop MFMA GEMM
     return wo_prefill_launch(kind, p.x, p.ldx, p.w, p.ldw, p.scale, p.zero, p.sz_dtype, p.group_steps, p.ngroups,
                              p.y, p.ldy, p.M, p.N, p.K, workspace, ws_bytes, kWoCounterBytes, st, name);
