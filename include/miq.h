@@ -118,9 +118,11 @@ int miq_fp8_dequantize(const uint8_t* q, const float* scale, int64_t rows, int64
  * Any M >= 1: decode kernels up to M = 64, a dequantize-in-the-K-loop MFMA GEMM above
  * (prefill), which splits K when the output has fewer 64 x 128 tiles than CUs, and, where
  * its 128 x 128..384 tiles fill the GPU (long prefill chunks), a GEMM that dequantizes
- * each weight block once per workgroup for the bf16 MFMA.
- * Workspace for the split-K reduction of the two weight-only GEMMs and for the last
- * kernel's packed activations and K-split partials. Its first 16384 bytes hold arrival
+ * each weight block once per workgroup for the bf16 MFMA. INT8 also has a kernel that splits
+ * K among a workgroup's wavefronts (decode batches and short prefills) and one for long
+ * chunks that streams both operands through LDS; neither uses the workspace.
+ * Workspace for the split-K reduction of the two weight-only GEMMs and for the
+ * dequantizing kernel's packed activations and K-split partials. Its first 16384 bytes hold arrival
  * counters that must be zero before the first call (zero the whole buffer once when
  * allocating it); every call leaves the whole workspace at zero again (counters, fp32
  * partials and packed activations alike). A workspace below this size for a long prefill call makes it take

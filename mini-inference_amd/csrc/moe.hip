@@ -1273,11 +1273,16 @@ size_t moe_block_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I)
          align_up((size_t)rows * 4) + align_up(moe_block_tiles(pairs, E) * sizeof(MoeTile)) +
          align_up((size_t)(pairs * 4)) + 256;
 }
+
+// what the streaming kernels and the routed align need: the least that a call may bring
+size_t moe_stream_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
+  const size_t rows = max_padded_rows(T * topk, E);
+  return moe_base_bytes(T, topk, E, H, I) + align_up(rows * 4) + align_up((rows + kTile - 1) / kTile * 4) + 256;
+}
 }  // namespace
 
 extern "C" size_t miq_moe_workspace_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
-  const size_t rows = max_padded_rows(T * topk, E);
-  const size_t bytes = moe_base_bytes(T, topk, E, H, I) + align_up(rows * 4) + align_up((rows + kTile - 1) / kTile * 4) + 256;
+  const size_t bytes = moe_stream_bytes(T, topk, E, H, I);
   return moe_block_ok(KIND_INT8, T, topk, E, H, I) ? std::max(bytes, moe_block_bytes(T, topk, E, H, I)) : bytes;
 }
 
@@ -1320,7 +1325,7 @@ int run_moe(int kind, const void* hidden, int64_t T, int64_t H, int64_t I, int64
   const int64_t wdiv = i8 ? 1 : 2;
   MIQ_REQUIRE(E * 2 * I * (H / wdiv) < 0x7fff0000LL && E * H * (I / wdiv) < 0x7fff0000LL,
               "%s: expert weights above 2 GiB", name);
-  const size_t need = miq_moe_workspace_bytes(T, topk, E, H, I);
+  const size_t need = moe_stream_bytes(T, topk, E, H, I);
   MIQ_REQUIRE(workspace != nullptr && workspace_bytes >= need, "%s: workspace of %zu bytes needed", name, need);
   MIQ_REQUIRE(((reinterpret_cast<uintptr_t>(workspace) & 15) | (reinterpret_cast<uintptr_t>(out) & 7)) == 0,
               "%s: workspace must be 16-byte and out 8-byte aligned", name);
@@ -1345,7 +1350,8 @@ int run_moe(int kind, const void* hidden, int64_t T, int64_t H, int64_t I, int64
   const size_t max_rows = max_padded_rows(T * topk, E);
   hipStream_t st = (hipStream_t)stream;
   MIQ_REQUIRE(!topk_ids || idx_dtype == MIQ_INT32 || idx_dtype == MIQ_INT64, "%s: topk_ids must be int32 or int64", name);
-  if ((topk_ids || (sorted_ids && expert_ids && num_padded)) && moe_block_ok(kind, T, topk, E, H, I)) {
+  if ((topk_ids || (sorted_ids && expert_ids && num_padded)) && moe_block_ok(kind, T, topk, E, H, I) &&
+      workspace_bytes >= moe_block_bytes(T, topk, E, H, I)) {
     const int64_t pairs = T * topk, rows = block_rows(pairs, E);
     char* at = static_cast<char*>(workspace);
     auto take = [&](size_t bytes) {

@@ -38,6 +38,8 @@ int wo_tile_launch(int kind, const uint16_t* x, int64_t ldx, const uint8_t* w, i
                    const void* zero, int sd, int group_steps, int64_t ngroups, uint16_t* y, int64_t ldy, int M,
                    int N, int K, void* pair, size_t pair_bytes, hipStream_t st, const char* name, bool& launched);
 
+size_t wo_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int weight_bits, bool with_wide);
+
 namespace {
 
 using namespace wo;
@@ -65,7 +67,9 @@ int run(int kind, const WoArgs& p, void* workspace, size_t ws_bytes, hipStream_t
               "%s: x must be 16-byte aligned with a row stride multiple of 8", name);
   MIQ_REQUIRE((reinterpret_cast<uintptr_t>(p.w) & 15) == 0, "%s: weights must be 16-byte aligned", name);
   MIQ_REQUIRE(p.ldx >= p.K && p.ldy >= p.N, "%s: bad strides", name);
-  if (kind == KIND_INT8) {  // decode batches (and some short prefills): the split kernel
+  // decode batches and some short prefills: the split kernel. It needs no workspace, but a call
+  // with less than the other kernels need keeps to them, which may refuse it.
+  if (kind == KIND_INT8 && workspace != nullptr && ws_bytes >= wo_gemm_workspace_bytes(p.M, p.N, p.K, 8, false)) {
     const WoSplitPlan pl = wo_split_plan(p.M, p.N, p.K, p.ldx);
     if (pl.mt != 0)
       return wo_split_launch(pl, p.x, p.ldx, p.w, p.scale, p.sz_dtype, p.y, p.ldy, p.M, p.N, p.K, st, name);

@@ -515,7 +515,10 @@ int wo_prefill_launch(int kind, const uint16_t* x, int64_t ldx, const uint8_t* w
                       const void* zero, int sd, int group_steps, int64_t ngroups, uint16_t* y, int64_t ldy, int64_t M,
                       int N, int K, void* workspace, size_t ws_bytes, size_t counter_bytes, hipStream_t st,
                       const char* name) {
-  if (kind == KIND_INT8 && wo_block_planned(M, N, K, ldx, wide_plan(M, N, K, ldw)))
+  // (the block kernel needs no workspace, but a call with less than this kernel needs keeps to it)
+  if (kind == KIND_INT8 && workspace != nullptr &&
+      ws_bytes >= wo_prefill_workspace_bytes(M, N, K, 8, counter_bytes, false) &&
+      wo_block_planned(M, N, K, ldx, wide_plan(M, N, K, ldw)))
     return wo_block_launch(x, ldx, w, scale, sd, y, ldy, M, N, K, st, name);
   // the wide kernel where it is planned and its workspace fits (the no-allocation entry
   // point's scratch may not hold it: then the prefill kernel)
