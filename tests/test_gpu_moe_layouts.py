@@ -39,3 +39,26 @@ def test_int4_scales_from_registers(T, H, I, E, k, sym):
                          None if sym else dn["zero"].to(DEV)).float().cpu()
     assert ((got - want).norm() / want.norm()).item() < 2e-2
     assert ((got - want).abs() <= 1e-2 + 2e-2 * want.abs()).all()
+
+
+@pytest.mark.parametrize("k", [1, 2, 7, 8, 9, 16, 17])
+@pytest.mark.parametrize("H", [128, 2048, 2176])
+def test_combine_order_of_many_tokens(k, H):
+    """The combine of large batches adds a token's slots in the same order as that of small
+    ones (bf16 after every addition, so another order gives other bytes): a call of 256 or 300
+    tokens equals calls of at most 100, with slots out of range for some tokens."""
+    from kernels.fused_moe import fused_moe_int4
+    print(f"[case] combine order k={k} H={H}", flush=True)
+    E, I = 20, 128
+    g = torch.Generator().manual_seed(23)
+    gu = O.int4_quantize_symmetric((torch.randn(E, 2 * I, H, generator=g) * 0.05).bfloat16(), 128)
+    dn = O.int4_quantize_symmetric((torch.randn(E, H, I, generator=g) * 0.05).bfloat16(), 128)
+    gq, gs, dq, ds = (x.to(DEV) for x in (gu["qweight"], gu["scale"], dn["qweight"], dn["scale"]))
+    hidden = torch.randn(300, H, generator=g).bfloat16().to(DEV)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(300)])
+    idx[::7, 0] = E
+    idx, w = idx.to(DEV), torch.rand(300, k, generator=g).bfloat16().to(DEV)
+    call = lambda a, b: fused_moe_int4(hidden[a:b], idx[a:b], w[a:b], gq, gs, None, dq, ds, None)  # noqa: E731
+    want = torch.cat([call(a, a + 100) for a in (0, 100, 200)])
+    assert torch.equal(call(0, 300), want)
+    assert torch.equal(call(0, 256), want[:256])
