@@ -394,10 +394,15 @@ bool fits(int64_t M, int64_t N, int64_t K, int64_t ldx) {
 // and, for a last round of at most 128 blocks (run as halves), one; a unit takes 0.83 us per
 // 64-k stage. It is compared with the wide plan's modelled time plus 4 us + 0.35 us per MB of
 // packed activations for its pack and clear launches; below the wide kernel's range (too few
-// tiles to fill the GPU) the prefill kernel stays. Measured block / before, us, MI355X: 19456 x
-// 2560 M = 1000 / 2048 / 4096: 110 / 185 / 360 against 129 / 238 / 439; 6144 x 2560 M = 700 /
-// 2048: 39 / 66 against 52 / 95; 12288 x 4096 M = 300 / 1000 / 4096: 58 / 95 / 335 against 69 /
-// 133 / 424; 2560 x 9728 M = 1000 / 2048: 122 / 124 against 78 (K splits, not taken) / 136.
+// tiles to fill the GPU) the prefill kernel stays. Where the line lies comes from a sweep of seven
+// N x K (2560 x 4096 .. 19456 x 2560 and 4096 x 12288) at M = 256 .. 3000, by the two models' ratio:
+//   wide without K splits, two or three row tiles: the block was faster at every ratio seen (0.8
+//     .. 1.33), by 8 to 37 % (19456 x 2560 M = 1024 / 2048 109 / 187 against 130 / 249 us, ratio
+//     1.02 / 0.90; 6144 x 2560 M = 1536 56 / 68, 1.29; 4096 x 12288 M = 3000 262 / 284, 1.24);
+//   one row tile or K splits: faster or even up to 1.13 (6144 x 2560 M = 512 34 / 37, 1.13; 2560 x
+//     9728 M = 2048 111 / 135, 0.99; 4096 x 12288 M = 1280 139 / 162, 1.07; 2560 x 4096 M = 1024
+//     47 / 47, 1.10), slower from 1.15 up (12288 x 4096 M = 256 50 / 47, 1.15; 2560 x 9728 M = 1536
+//     / 1024 106 / 101, 1.32, and 103 / 77, 1.77).
 bool wo_block_planned(int64_t M, int64_t N, int64_t K, int64_t ldx, const WidePlan& wide) {
   const Tuning& t = tuning();
   if (t.wo_block == 0 || !fits(M, N, K, ldx)) return false;
@@ -407,7 +412,8 @@ bool wo_block_planned(int64_t M, int64_t N, int64_t K, int64_t ldx, const WidePl
   const int64_t T = ((M + 255) / 256) * ((N + 255) / 256), rest = T % 256;
   const int64_t units = 2 * (T / 256) + (rest == 0 ? 0 : rest <= 128 ? 1 : 2);
   const double block_us = 4.0 + 0.83 * (double)(units * (K / kBK));
-  return block_us < 0.97 * (wide.us + 4.0 + 0.35e-6 * (double)wide.pack_bytes);
+  const double wide_us = wide.us + 4.0 + 0.35e-6 * (double)wide.pack_bytes;
+  return block_us < (wide.S == 1 && wide.mt >= 2 ? 1.35 : 1.14) * wide_us;
 }
 
 int wo_block_launch(const uint16_t* x, int64_t ldx, const uint8_t* w, const void* scale, int sd, uint16_t* y, int64_t ldy,
