@@ -19,6 +19,7 @@
 
 #include <mutex>
 
+#include "fp8_plan.h"
 #include "fp8_split.h"
 #include "miq_common.h"
 
@@ -247,12 +248,9 @@ fp8_gemm32_kernel(const uint8_t* __restrict__ A, const float* __restrict__ sa,
   }
   const int m0 = tm * BM, n0 = tn * BN;
 
-  // this lane's part of every load: row lane / 4 of the 16, global chunk (lane & 3) ^
-  // ((lane >> 4) & 3); rows past M or N read zeros (the descriptor's size)
+  // rows past M or N read zeros: their offsets lie outside the buffers (fp8_plan.h)
   const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(A), 0, M * K, 0x00020000);
   const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(B), 0, N * K, 0x00020000);
-  const int lrow = lane >> 2, lchunk = (lane & 3) ^ ((lane >> 4) & 3);
-  const int voffA = (m0 + lrow) * K + lchunk * 16, voffB = (n0 + lrow) * K + lchunk * 16;
   typedef __attribute__((address_space(3))) void* lds_ptr;
   // WV = 4: wavefront w issues A loads 4 w .. 4 w + 3 and B loads 3 w .. 3 w + 2 of each
   // stage; WV = 8: A loads 2 w, 2 w + 1 and B loads 2 w, 2 w + 1 (w < 4) or 4 + w (w >= 4)
@@ -261,18 +259,22 @@ fp8_gemm32_kernel(const uint8_t* __restrict__ A, const float* __restrict__ sa,
   const int qa0 = wv * nA;
   const int nB = WV == 4 ? 3 : (wv < 4 ? 2 : 1);
   const int qb0 = WV == 4 ? wv * 3 : (wv < 4 ? wv * 2 : 4 + wv);
+  int voffA[4], voffB[3];  // (the four-wavefront layout fills them)
+#pragma unroll
+  for (int u = 0; u < nA; ++u) voffA[u] = fp8_large_offset(m0, qa0 + u, lane, M, K);
+#pragma unroll
+  for (int u = 0; u < nBmax; ++u) voffB[u] = fp8_large_offset(n0, qb0 + u, lane, N, K);
   auto issue = [&](int st, int slot) {  // stage st into ring slot `slot`
     uint8_t* base = smem + slot * kStage;
     const int k0 = st * BK32;
 #pragma unroll
     for (int u = 0; u < nA; ++u)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (lds_ptr)(base + (qa0 + u) * 1024), 16, voffA + k0,
-                                               (qa0 + u) * 16 * K, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (lds_ptr)(base + (qa0 + u) * 1024), 16, voffA[u], k0, 0, 0);
 #pragma unroll
     for (int u = 0; u < nBmax; ++u)
       if (u < nB)  // uniform
         __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (lds_ptr)(base + BM * kRowBytes + (qb0 + u) * 1024), 16,
-                                                 voffB + k0, (qb0 + u) * 16 * K, 0, 0);
+                                                 voffB[u], k0, 0, 0);
   };
 
   f32x16 acc[kTM][kTN];
@@ -461,7 +463,7 @@ extern "C" int miq_fp8_gemm(const uint8_t* xq, const float* x_scale, const uint8
   hipStream_t st = (hipStream_t)stream;
   uint16_t* yy = static_cast<uint16_t*>(y);
   // kernels that address the operands through buffer descriptors take operands below 2 GiB
-  const bool buffers = !tuning().fp8_old && M * K < 0x7fffff00LL && N * K < 0x7fffff00LL;
+  const bool buffers = !tuning().fp8_old && M * K < kFp8BufferLimit && N * K < kFp8BufferLimit;
   // The kernel of least modelled time (us, MI355X). Large tiles: 5 us + 0.8 us per 64-k stage for
   // every round of 256 tiles, 0.65 us a stage when half the CUs are idle (2048 x 6144 x 2560: 37
   // us, x 9728: 118; 2048 x 2560 x 9728: 100). 128 x 128 tiles, two workgroups per CU: 10 us +
