@@ -2,10 +2,10 @@
 //
 //   y[m, n] = sum_k x[m, k] * W[n, k],  x bf16 [M, K],  W int8 [N, K] or int4 [N, K/2]
 //
-// Argument checks live here. INT8 batches of 17 to 64 rows (5 to 16 where its tiles are small) run
-// the split kernel (wo_split.hip). Otherwise up to 16 rows whose activations fit LDS run the
-// one-tile-per-workgroup kernel (wo_tile.hip); the rest the streamed split-K kernel
-// (wo_stream.hip).
+// Argument checks live here. INT8 batches of 5 rows and more run the split kernel (wo_split.hip) where
+// its tiles are about one per CU and K is not too deep for them. Otherwise up to 16 rows whose
+// activations fit LDS run the one-tile-per-workgroup kernel (wo_tile.hip); the rest the streamed
+// split-K kernel (wo_stream.hip).
 #include <algorithm>
 #include <mutex>
 

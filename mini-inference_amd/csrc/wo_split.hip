@@ -234,11 +234,51 @@ void go(const WoSplitParams& p, int sd, hipStream_t st) {
 //   2560 x 4096    7.8/10.3   8.1/11.5   10.1/19.9  10.2/24.6  11.4/30.2
 //   12288 x 4096   14.9/16.2  15.2/17.4  16.9/23.5  19.5/29.0  23.0/33.0
 //   19456 x 2560   18.0/16.7  18.1/18.2  20.1/22.2  22.6/27.6  26.2/33.0
-// so it takes M = 17 .. 64, and 5 .. 16 where the tiles are at most 48 weight rows. Past 64 rows it
-// takes the calls whose modelled time (4 us + the bytes at 46 KB per us + 0.1 us per MB of
-// weights) is below what the prefill kernels were never seen under at that depth of K: 26 us, or
-// 17 us below 20 k-steps (M = 128: 6144 x 2560 15.4 against 33.7 us, 2560 x 4096 13.1 against 28.6,
-// 1024 x 1024 5.2 against 19.3; 19456 x 2560 44.1 against 37.9, not taken).
+// The rule's lines come from two more sweeps, of this kernel against the others over N = 512 ..
+// 151936, K = 512 .. 19456 and M = 5 .. 256 (5200 calls): inside the lines it was nowhere slower by
+// more than 3 %. Each gives the deepest K that a tile shape pays for: a workgroup walks all of K,
+// where the streamed kernel gives a deep K to several workgroups, so narrow tiles (few weights
+// per activation) lose first. Split / other kernel, us:
+//   M = 5 .. 16:  5120 x 12288 M = 8 20.7/17.6, 512 x 16384 13.9/11.1; 12288 x 4096 M = 8 16.2/15.2;
+//     M = 5 (a plan of one weight tile is the only one that pays) 6144 x 2560 8.4/7.4;
+//   16-row tiles by 64 or 80 weights:  8192 x 4096 M = 17 14.9/19.0, x 8192 25.4/23.6; 6144 x 6144 M
+//     = 36 23/24, x 14336 M = 40 47.3/39.9;
+//   32-row tiles by 64 or 80:  20480 x 3072 M = 18 22.7/21.2; 9728 x 9728 M = 36 41.9/38.2, M = 60
+//     faster.
+// Tiles of 32 rows or more fill a CU's LDS, so a second tile waits for the first, whereas the
+// other kernels' time grows with the weights alone:
+//   two tiles per CU:  by 48 weights 24576 x 2560 M = 32 20.9/26.8; by 64 28672 x 1024 13.7/17.4,
+//     32768 x 2048 M = 17 22.6/20.5, 28672 x 8192 M = 48 72/80; by 80 40960 x 2560 M = 17
+//     37.4/31.2, x 8192 M = 48 91/130;
+//   three:  49152 x 1024 M = 64 33.5/25.6, x 4096 M = 40 73/71, x 8192 106/126;
+//   more (a vocabulary's projection):  151936 x 2560 M = 17 137/83, 50304 x 2048 M = 64 58/45.
+// Past 64 rows it takes the calls whose modelled time (4 us + the bytes at 46 KB per us + 0.1 us
+// per MB of weights) is below what the prefill kernels were never seen under at that depth of K: 26
+// us, or 17 us below 20 k-steps (M = 128: 6144 x 2560 15.4 against 33.7 us, 2560 x 4096 13.1
+// against 28.6, 1024 x 1024 5.2 against 19.3; 19456 x 2560 44.1 against 37.9, not taken), and with
+// a second tile per CU only from 16 k-steps up (M = 96, 12288 x 512 13.8 against 11.3, x 1024 17.7
+// against 16.1, x 2560 27.9 against 35.8).
+static bool split_is_faster(const WoSplitPlan& pl, int64_t per_cu, double bytes, int64_t M, int64_t N, int64_t K) {
+  const int64_t steps = K / kStepK;
+  if (M <= 4 || steps > 128) return false;
+  if (M > 64) {
+    const double us = 4.0 + bytes / 46e3 + 1e-7 * (double)N * (double)K;
+    return us < (steps >= 20 ? 26.0 : 17.0) && (per_cu == 1 || steps >= 16);
+  }
+  if (M < 8) return (pl.nt == 1 && steps <= 64) || (M >= 6 && pl.nt <= 3 && steps <= (pl.nt == 2 ? 32 : 24));
+  if (M <= 16) {
+    if (pl.nt <= 2) return steps <= (pl.nt == 1 ? 80 : 64);
+    return pl.nt == 3 && (per_cu > 1 || M >= 12 || steps <= 24 || steps >= 48);
+  }
+  if (per_cu == 1) {
+    if (pl.nt <= 3 || pl.mt >= 3) return true;
+    if (pl.mt == 1) return steps <= (M <= 24 ? 32 : 64);
+    return M > 48 || steps <= (pl.nt == 4 ? 80 : M <= 24 ? 20 : 32);
+  }
+  if (per_cu == 2 && (pl.nt <= 3 || (pl.nt == 4 && steps <= 12) || (pl.nt == 5 && steps >= 32))) return true;
+  return M > 24 && steps >= 64 && (per_cu == 2 || (per_cu == 3 && pl.nt <= 4));
+}
+
 WoSplitPlan wo_split_plan(int64_t M, int64_t N, int64_t K, int64_t ldx) {
   WoSplitPlan best;
   const Tuning& t = tuning();
@@ -248,7 +288,6 @@ WoSplitPlan wo_split_plan(int64_t M, int64_t N, int64_t K, int64_t ldx) {
                           t.wo_int8_tile2_min_m || t.wo_gemv_max_m >= 0 || t.wo_prefill_min_m != 65 || t.wo_prefill_s > 0 ||
                           t.wo_wide_mt >= 0 || t.wo_wide_s > 0 || t.wo_block == 1))
     return best;
-  if (t.wo_split != 1 && M <= 4) return best;
   double bytes = 0.0;
   int64_t per_cu = 0;
   for (int mt = 1; mt <= 4; ++mt)
@@ -263,9 +302,7 @@ WoSplitPlan wo_split_plan(int64_t M, int64_t N, int64_t K, int64_t ldx) {
     }
   const int64_t steps = K / kStepK;
   best.nw = per_cu == 1 && steps >= 32 && best.nt <= (best.mt == 1 ? 3 : best.mt == 2 ? 2 : 0) ? 8 : 4;
-  if (t.wo_split == 1) return best;
-  const double us = 4.0 + bytes / 46e3 + 1e-7 * (double)N * (double)K;
-  if ((M <= 16 && best.nt > 3) || (M > 64 && us >= (steps >= 20 ? 26.0 : 17.0))) best.mt = 0;
+  if (t.wo_split != 1 && !split_is_faster(best, per_cu, bytes, M, N, K)) best.mt = 0;
   return best;
 }
 

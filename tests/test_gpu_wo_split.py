@@ -50,7 +50,15 @@ def test_w8a16_split(M, N, K, sdt, miq_env):
 
 
 @pytest.mark.parametrize("M,N,K,split", [(64, 2560, 4096, True), (8, 6144, 2560, True), (8, 19456, 2560, False),
-                                         (4, 6144, 2560, False), (128, 1024, 1024, True), (128, 19456, 2560, False)])
+                                         (4, 6144, 2560, False), (128, 1024, 1024, True), (128, 19456, 2560, False),
+                                         # one, two and three tiles per CU; a vocabulary's projection
+                                         (64, 20480, 512, True), (64, 24576, 512, True), (48, 32768, 1024, True),
+                                         (64, 40960, 512, False), (64, 40960, 4096, True), (17, 49152, 512, False),
+                                         (32, 50304, 2048, False),
+                                         # a deep K on narrow tiles; five to seven rows; past 64 rows
+                                         (40, 6144, 14336, False), (17, 8192, 4096, True), (16, 2560, 12288, False),
+                                         (12, 2560, 9728, True), (5, 6144, 1024, False), (6, 6144, 1024, True),
+                                         (96, 12288, 512, False), (96, 12288, 2560, True)])
 def test_w8a16_split_is_the_planned_kernel(M, N, K, split, miq_env):
     """Both sides of the dispatch's lines: the call gives the bytes of the kernel the rule names."""
     from kernels import quant_ops as ops
