@@ -1274,7 +1274,8 @@ int64_t block_rows(int64_t pairs, int64_t E) { return pairs + std::min(E, pairs)
 bool moe_block_ok(int kind, int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
   const int64_t pairs = T * topk;
   const int force = tuning().moe_block;
-  if (kind != KIND_INT8 || force == 0 || pairs >= 65536 || moe_group_lds(pairs, E) > (size_t)150 * 1024) return false;
+  if (kind != KIND_INT8 || force == 0 || pairs < 1 || E < 1 || pairs >= 65536) return false;
+  if (moe_group_lds(pairs, E) > (size_t)150 * 1024) return false;
   if (!moe_block_fits(T, topk, E, H, I, block_rows(pairs, E))) return false;
   return force == 1 || pairs > 16 * E;
 }

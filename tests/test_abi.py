@@ -60,6 +60,13 @@ def test_workspace_sizes():
     assert lib.miq_moe_workspace_bytes(64, 8, 64, 2048, 1024) >= 64 * 8 * 2048 * 4
 
 
+@pytest.mark.parametrize("T,k,E", [(4, 2, 0), (0, 2, 8), (0, 0, 0), (300, 2, 0)])
+def test_workspace_query_of_empty_layers(T, k, E):
+    """A layer without experts or tokens has a size too (the layer itself refuses it)."""
+    from kernels import _lib
+    assert 0 <= _lib.load().miq_moe_workspace_bytes(T, k, E, 256, 128) < 1 << 20
+
+
 def test_cpu_tensors_are_refused():
     from engine.quantization import get_method
     from kernels.paged_attention import paged_decode_attention
