@@ -196,6 +196,13 @@ moe_align_chunks_kernel(const void* __restrict__ ids, int dtype, int num_pairs, 
   }
 }
 
+// LDS tables of that kernel, and their largest size
+constexpr int64_t kAlignChunkBytes = 64 * 1024;
+int64_t align_chunk_ints(int64_t num_pairs, int64_t E) {
+  const int64_t nch = (num_pairs + 63) / 64;
+  return 2 * E + 1 + nch * E + nch * 128;
+}
+
 // The grouping of the block GEMMs (wo_block.hip) in one workgroup: experts padded to kGroupRows
 // rows, and the list of row tiles (up to kMoeTileRows rows; an expert's rows spread evenly over
 // its tiles). Ranks inside an expert come from ballots as above, and are formed again when the
@@ -1266,18 +1273,54 @@ void launch_experts(const MoeParams& p, bool hz, int sd, dim3 gu_grid, dim3 dn_g
 }
 
 // Whether a routed layer takes the block GEMMs: int8 experts with more than 16 pairs each on
-// average. The streaming kernels read an expert's weights once per 16 rows; the block GEMMs once
-// per 160, with every MFMA fragment used by up to 160 rows. OLMoE layer, MI355X, T = 64 / 128 /
-// 144 / 256 / 512 / 1000 / 2000: streaming 82 / 103 / 136 / 185 / 283 / 547 / 987 us, block 101 /
-// 111 / 107 / 115 / 135 / 172 / 311 us (the weights alone: 86 us at the copy rate).
+// average, where the modelled time of the block GEMMs is the lower one. The streaming kernels
+// read an expert's weights once per 16 rows, the block GEMMs once per 160, with every MFMA
+// fragment used by up to 160 rows; but a block is a whole row tile by 256 or 512 columns over all
+// of K, so a layer of few experts or narrow ones gives few of them, whose stages and epilogues
+// are the layer's time. Both models take the pairs as spread evenly over the experts; fitted on
+// 228 layers (20 sizes, E = 1 .. 300, H = 256 .. 5120, I = 128 .. 14336, 17 .. 1600 pairs per
+// expert, MI355X), the rule picks the faster kernels or ones within 5 % of them in 216, and is never
+// on the block GEMMs where they are slower. Streaming / block, us:
+//   E = 64, top 8, 2048 x 1024 (OLMoE), T = 136 / 256 / 512 / 1024: 143/105, 183/110, 278/132, 552/175;
+//   E = 8, top 2, 4096 x 14336, T = 68 / 128 / 512: 366/456, 591/479, 1632/636;
+//   E = 8, top 1, 2048 x 8192, T = 136 / 512: 136/194, 265/232;
+//   E = 16, top 4, 1024 x 512, T = 128 / 512 / 1600: 30/41, 58/78, 126/87;
+//   E = 1, 2048 x 4096, T = 128 / 1600: 61/135, 300/175;  E = 4, 256 x 128, T = 512: 20/48.
+// Pairs that crowd on some of the experts make the longest block longer: where the last sixth of
+// the experts had almost none, narrow layers near the line lost (E = 64, top 8, 1024 x 512, T = 256
+// 59/78) and the wide ones did not.
 int64_t block_rows(int64_t pairs, int64_t E) { return pairs + std::min(E, pairs) * (kGroupRows - 1); }
+
+double moe_stream_us(int64_t pairs, int64_t E, int64_t H, int64_t I) {
+  const double depth = 17.0 + 0.77 * (double)((H + I) / kStepK);  // a lone workgroup's k-steps
+  // each 16-row tile reads its expert's weights, at 6.6 TB/s
+  const double tiles = (double)pairs / kTile + 0.5 * (double)E;
+  const double bytes = tiles * 3.0 * (double)H * (double)I / 6.6e6;
+  double us = std::max(depth, bytes) + 0.44 * std::min(depth, bytes);
+  if (pairs > kRtPairs || E > kRtExperts)  // moe_align's launch, past its chunk tables one wavefront per expert
+    us += align_chunk_ints(pairs, E) * 4 <= kAlignChunkBytes ? 7.0 : 1.8e-4 * (double)pairs * (double)E;
+  return us;
+}
+
+double moe_block_us(int64_t pairs, int64_t E, int64_t H, int64_t I) {
+  const int64_t per = (pairs + E - 1) / E, tiles = (per + kMoeTileRows - 1) / kMoeTileRows;  // of one expert
+  const double mt = (double)((per + 32 * tiles - 1) / (32 * tiles));                          // 32-row blocks of one
+  double us = 12.0;  // grouping and combine
+  auto gemm = [&](int64_t K, int64_t column_blocks, double weights) {
+    const double rounds = (double)((E * tiles * column_blocks + 255) / 256);
+    us += std::max(rounds * ((double)(K / 64) * (0.9 + 0.15 * mt) + 1.3 + 3.3 * mt), weights / 4.3e6);
+  };
+  gemm(H, (I + 255) / 256, 2.0 * (double)E * (double)H * (double)I);
+  gemm(I, (H + 511) / 512, (double)E * (double)H * (double)I);
+  return us;
+}
+
 bool moe_block_ok(int kind, int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
   const int64_t pairs = T * topk;
   const int force = tuning().moe_block;
   if (kind != KIND_INT8 || force == 0 || pairs < 1 || E < 1 || pairs >= 65536) return false;
-  if (moe_group_lds(pairs, E) > (size_t)150 * 1024) return false;
-  if (!moe_block_fits(T, topk, E, H, I, block_rows(pairs, E))) return false;
-  return force == 1 || pairs > 16 * E;
+  if (moe_group_lds(pairs, E) > (size_t)150 * 1024 || !moe_block_fits(T, topk, E, H, I, block_rows(pairs, E))) return false;
+  return force == 1 || (pairs > 16 * E && 1.05 * moe_block_us(pairs, E, H, I) < moe_stream_us(pairs, E, H, I));
 }
 
 size_t max_padded_rows(int64_t num_pairs, int64_t E) { return (size_t)(num_pairs + E * (kTile - 1)); }
@@ -1296,9 +1339,8 @@ extern "C" int miq_moe_align(const void* topk_ids, int idx_dtype, int64_t num_pa
               (long long)block_m);
   const int64_t max_padded = num_pairs + E * (block_m - 1);
   const int64_t max_blocks = (max_padded + block_m - 1) / block_m;
-  const int64_t nch = (num_pairs + 63) / 64;
-  const int64_t chunk_ints = 2 * E + 1 + nch * E + nch * 128;
-  if (chunk_ints * 4 <= 64 * 1024 && !tuning().moe_align_scan) {
+  const int64_t chunk_ints = align_chunk_ints(num_pairs, E);
+  if (chunk_ints * 4 <= kAlignChunkBytes && !tuning().moe_align_scan) {
     hipLaunchKernelGGL(moe_align_chunks_kernel, dim3(1), dim3(1024), (size_t)chunk_ints * sizeof(int),
                        (hipStream_t)stream, topk_ids, idx_dtype, (int)num_pairs, (int)E, (int)block_m,
                        (int)max_padded, (int)max_blocks, sorted_ids, expert_ids, num_padded);

@@ -99,13 +99,15 @@ def test_int8_moe_block(counts, H, I, wdtype, ids, miq_env):
     assert ((got - loop).abs() <= 1e-2 + 2e-2 * loop.abs()).all()
 
 
-@pytest.mark.parametrize("T,E,k", [(65, 8, 2), (700, 40, 3), (1100, 8, 8), (40, 300, 4)])
-def test_int8_moe_block_equals_streaming(T, E, k, miq_env):
+@pytest.mark.parametrize("T,E,k,H,I,planned", [(65, 8, 2, 256, 128, False), (700, 40, 3, 256, 128, False),
+                                               (1100, 8, 8, 256, 128, False), (40, 300, 4, 256, 128, False),
+                                               (1500, 300, 4, 256, 128, True), (600, 16, 8, 1024, 512, True)])
+def test_int8_moe_block_equals_streaming(T, E, k, H, I, planned, miq_env):
     """More experts than a wavefront or than threads per segment, more than 128 chunks of pairs
-    (T = 1100, k = 8), and the dispatch rule's default: block and streaming kernels place the
-    same pairs, so tokens agree to the layer's bound, and repeated calls to the byte."""
-    print(f"[case] int8 moe block vs streaming T={T} E={E} k={k}", flush=True)
-    H, I = 256, 128
+    (T = 1100, k = 8), and the dispatch rule's default on both sides of its line: block and
+    streaming kernels place the same pairs, so tokens agree to the layer's bound, and repeated
+    calls to the byte."""
+    print(f"[case] int8 moe block vs streaming T={T} E={E} k={k} H={H} I={I}", flush=True)
     gu, dn, g = _layer(E, H, I, seed=43)
     hidden = torch.randn(T, H, generator=g).to(torch.bfloat16)
     idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)])
@@ -116,5 +118,5 @@ def test_int8_moe_block_equals_streaming(T, E, k, miq_env):
     miq_env("MIQ_MOE_BLOCK", "1")
     block = _run(hidden, idx, w, gu, dn)
     assert torch.equal(block, _run(hidden, idx, w, gu, dn))
-    assert torch.equal(default, block if T * k > 16 * E else stream)
+    assert torch.equal(default, block if planned else stream) and not torch.equal(block, stream)
     assert ((block - stream).abs() <= 1e-2 + 2e-2 * stream.abs()).all()

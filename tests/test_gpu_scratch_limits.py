@@ -22,6 +22,7 @@ def test_int8_moe_takes_the_streaming_kernels_scratch(routed, miq_env):
     hidden = torch.randn(T, H, generator=g).bfloat16().to(DEV)
     idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).to(DEV)
     w = torch.rand(T, k, generator=g).bfloat16().to(DEV)
+    miq_env("MIQ_MOE_BLOCK", "1")
     full = L.load().miq_moe_workspace_bytes(T, k, E, H, I)
     miq_env("MIQ_MOE_BLOCK", "0")
     small = L.load().miq_moe_workspace_bytes(T, k, E, H, I)
