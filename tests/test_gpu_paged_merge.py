@@ -1,6 +1,7 @@
 """The merge of the partitions of paged decode attention, at the partition counts where its
-loops end: none, one, a workgroup's rows in flight (16 or 64) and one more, and past the 512
-partitions whose weights are formed at once.
+loops end: none, one, the most that one thread per column holds (4, 8 and 16) and one more, a
+workgroup's rows in flight (64) and one more, and past the 512 partitions whose weights are
+formed at once.
 
 Each head puts about half of its probability on one token of one partition, so a partition that
 is left out, added twice or given another's weight moves that head's output by about half a
@@ -16,8 +17,9 @@ DEV = "cuda"
 H, D, PAGE, PART = 8, 128, 16, 128
 
 
-@pytest.mark.parametrize("lens", [[0, 1, 127, 128, 129, 2047, 2048], [0, 5, 128 * 16 + 1, 128 * 64, 128 * 64 + 1],
-                                  [128 * 511 + 3, 130], [128 * 519 + 3, 0],
+@pytest.mark.parametrize("lens", [[0, 3, 128], [0, 1, 129, 385, 512], [0, 129, 513], [1, 500, 1024], [0, 1025, 300],
+                                  [0, 1, 127, 128, 129, 2047, 2048], [0, 5, 128 * 16 + 1, 128 * 64, 128 * 64 + 1],
+                                  [128 * 16 + 1, 0], [128 * 511 + 3, 130], [128 * 519 + 3, 0],
                                   [0, 2049, 128 * 33] + [129] * 125])
 @pytest.mark.parametrize("unaligned", [False, True])
 def test_merge_adds_every_partition_once(lens, unaligned):
