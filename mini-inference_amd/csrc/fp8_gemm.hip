@@ -13,7 +13,6 @@
 // with the same (lane / 16) * 32 byte offset along k, so whatever order the hardware
 // assigns to those 32 bytes inside the instruction, A and B agree and the sum over k is
 // the dot product.
-#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -464,27 +463,14 @@ extern "C" int miq_fp8_gemm(const uint8_t* xq, const float* x_scale, const uint8
   uint16_t* yy = static_cast<uint16_t*>(y);
   // kernels that address the operands through buffer descriptors take operands below 2 GiB
   const bool buffers = !tuning().fp8_old && M * K < kFp8BufferLimit && N * K < kFp8BufferLimit;
-  // The kernel of least modelled time (us, MI355X). Large tiles: 5 us + 0.8 us per 64-k stage for
-  // every round of 256 tiles, 0.65 us a stage when half the CUs are idle (2048 x 6144 x 2560: 37
-  // us, x 9728: 118; 2048 x 2560 x 9728: 100). 128 x 128 tiles, two workgroups per CU: 10 us +
-  // 1.4 us per 128-k step for every 512. Split tiles: fp8_split_plan. At N = 19456, K = 2560 the
-  // 128 x 128 tiles used to take every M (no multiple of 192): M = 300 / 512 / 1000 / 2048 46 / 81
-  // / 122 / 215 us, on large tiles 33 / 37 / 71 / 142; at M = 200 the two meet (46 us).
-  const double steps = (double)(K / BK);
-  const int64_t big = ((M + 255) / 256) * ((N + 191) / 192), small = ((M + 127) / 128) * ((N + 127) / 128);
-  const double t_small = (double)((small + 511) / 512) * (10.0 + 1.4 * steps);
-  // (the large-tile kernel stores 16-byte pieces of y rows)
-  const bool can_big = buffers && N % 8 == 0 && ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
-  const double t_big = can_big ? (double)((big + 255) / 256) * (5.0 + (big <= 128 ? 1.3 : 1.6) * steps) : 1e30;
-  if (buffers) {
-    const Fp8SplitPlan pl = fp8_split_plan(M, N, K);
-    if (pl.us < std::min(t_small, t_big))
-      return fp8_split_launch(pl, xq, x_scale, wq, w_scale, yy, ldy, M, N, K, st);
+  const Fp8Plan pl = fp8_plan(M, N, K, buffers, ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0);
+  switch (pl.kernel) {
+    case Fp8Kernel::kSplit: return fp8_split_launch(pl.split, xq, x_scale, wq, w_scale, yy, ldy, M, N, K, st);
+    case Fp8Kernel::kLarge: return launch32<256, 192>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
+    case Fp8Kernel::kPrevious:
+      return launch<256, 192, 4, 2>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
+    default: return launch<128, 128, 2, 2>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
   }
-  if (t_big < t_small) return launch32<256, 192>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
-  if (M >= 1024 && N % 192 == 0)
-    return launch<256, 192, 4, 2>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
-  return launch<128, 128, 2, 2>(xq, x_scale, wq, w_scale, yy, ldy, (int)M, (int)N, (int)K, st);
 }
 
 extern "C" size_t miq_fp8_linear_workspace_bytes(int64_t M, int64_t K) {

@@ -6,19 +6,17 @@
 // A workgroup owns a tile of 16 MT activation rows x 16 NT weight rows and its NW wavefronts
 // split K between them: each multiplies the whole tile over its own k-steps of 128, with every
 // operand loaded straight from memory into registers (no LDS staging, no barrier in the K loop),
-// D k-steps ahead; the wavefronts' fp32 tiles are then added in LDS in wavefront order. A
-// single row tile of N = 6144 so becomes 384 workgroups x 4 wavefronts of 5 k-steps instead
-// of 48 workgroups that walk all 20 k-steps one after another.
-#include <algorithm>
-
+// D k-steps ahead; the wavefronts' fp32 tiles are then added in LDS in wavefront order. 16 rows
+// by N = 6144, K = 2560 so become 192 workgroups of 8 wavefronts with two or three k-steps each,
+// instead of 48 workgroups that walk all 20 k-steps one after another.
 #include "fp8_split.h"
 #include "miq_common.h"
 
 namespace miq {
 namespace {
 
-constexpr int kStep = 128;           // k per MFMA step
-constexpr int kOutF = 0x7ffffff0;    // outside every buffer: the load returns zeros
+constexpr int kStep = kFp8Step;  // k per MFMA step
+constexpr int kOutF = kFp8Outside;
 
 struct SplitParams {
   const uint8_t* x;
@@ -166,37 +164,6 @@ void go(const SplitParams& p, hipStream_t st) {
 }
 
 }  // namespace
-
-// Tile sizes, wavefronts and modelled time of a call. The kernel runs at the rate at which a CU pulls
-// operands from L2, so the plan takes the tile that needs the fewest bytes on the busiest CU
-// (tiles per CU, rounded up, times the tile's rows; activation rows, read 64 bytes at a time,
-// weigh 1.3 times the weights' whole lines), and fewer wavefronts per workgroup where a CU
-// holds several workgroups. Chosen from a sweep on MI355X of every (MT, NT, NW) below over N x
-// K = 6144 x 2560, 2560 x 9728, 19456 x 2560, 2560 x 4096 and 1024 x 1024 at M = 1 .. 1000: the
-// plan is within 10 % of the fastest tile. Split against 128 x 128 tiles, us (rotating weight
-// copies): 6144 x 2560 M = 1 / 16 / 64 / 256 / 512: 6 / 7 / 11 / 21 / 31 against 31 / 33 / 40 /
-// 42 / 41; 2560 x 9728: 8 / 11 / 17 / 31 / 54 against 101 / 102 / 110 / 113 / 110. Modelled
-// time (miq_fp8_gemm compares it with the other kernels'): 4 us, those bytes at 41 (K = 2560) to
-// 59 KB (K = 9728) per us, and 0.1 us per MB of weights.
-Fp8SplitPlan fp8_split_plan(int64_t M, int64_t N, int64_t K) {
-  static const int kTiles[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {4, 2}, {4, 4}};
-  Fp8SplitPlan best;
-  double best_bytes = 0.0;
-  for (const auto& t : kTiles) {
-    const int64_t items = ((M + 16 * t[0] - 1) / (16 * t[0])) * ((N + 16 * t[1] - 1) / (16 * t[1]));
-    const int64_t per_cu = (items + 255) / 256;
-    const double bytes = (double)per_cu * (double)K * 16.0 * (1.3 * t[0] + t[1]);
-    if (best.mt != 0 && bytes >= best_bytes) continue;
-    best_bytes = bytes;
-    best.mt = t[0];
-    best.nt = t[1];
-    best.nw = per_cu == 1 ? 8 : per_cu <= 3 ? 4 : 2;
-  }
-  const int64_t steps = K / kStep;
-  while (best.nw > 2 && steps < 2 * best.nw) best.nw /= 2;
-  best.us = 4.0 + best_bytes / (34e3 + 330.0 * (double)std::min<int64_t>(steps, 76)) + 1e-7 * (double)N * (double)K;
-  return best;
-}
 
 // Launches the planned tile; operands below 2 GiB, K a multiple of 128.
 int fp8_split_launch(const Fp8SplitPlan& pl, const uint8_t* xq, const float* xs, const uint8_t* wq, const float* ws,

@@ -45,7 +45,12 @@ extern "C" long faults(int rows, int K, int tile, int loads, int split) {
       }
   return bad;
 }
+
+extern "C" int kernel(long M, long N, long K, int buffers, int rows16) {
+  return (int)fp8_plan(M, N, K, buffers, rows16).kernel;
+}
 """
+SPLIT, LARGE, SMALL, PREVIOUS = range(4)
 
 
 @pytest.fixture(scope="module")
@@ -57,6 +62,7 @@ def lib(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, src, "-o", so], check=True)
     out = ctypes.CDLL(so)
     out.faults.restype = ctypes.c_long
+    out.kernel.argtypes = [ctypes.c_long] * 3 + [ctypes.c_int] * 2
     return out
 
 
@@ -84,3 +90,47 @@ def test_the_check_finds_rows_in_the_scalar_offset(lib, tile, loads):
     tile (a planted mistake)."""
     for rows in (1, 65, 129, 175):
         assert lib.faults(rows, 2560, tile, loads, 1) > 0, rows
+
+
+# (M, N, K) -> the kernel that measures fastest there, of every size by more than 5 %
+FASTEST = {(1, 6144, 2560): SPLIT, (64, 2560, 9728): SPLIT, (512, 2560, 4096): SPLIT, (100, 2560, 4096): SPLIT,
+           (200, 19456, 2560): LARGE, (300, 19456, 2560): LARGE, (1000, 19456, 2560): LARGE,
+           (2048, 6144, 2560): LARGE, (1280, 6144, 4096): LARGE, (2560, 6144, 4096): LARGE, (1280, 12288, 4096): LARGE,
+           (1536, 4608, 9728): LARGE, (2048, 3264, 3200): LARGE, (2560, 2560, 4096): LARGE, (1024, 8192, 8192): LARGE}
+
+
+def test_the_fastest_kernel_is_chosen(lib):
+    for size, kernel in FASTEST.items():
+        assert lib.kernel(*size, 1, 1) == kernel, size
+
+
+def test_the_large_tiles_replacements_stay_with_calls_they_cannot_take(lib):
+    """Over a grid of sizes: a call with 16-byte output rows and operands in reach of buffer
+    descriptors runs on split or large tiles, whatever divides N; one without runs on split or
+    on register-staged tiles, of 256 x 192 only where it always did."""
+    seen = set()
+    for M in list(range(1, 66, 8)) + list(range(65, 4200, 61)):
+        for N in (16, 192, 200, 1008, 1920, 2560, 3264, 4608, 6144, 12288, 19456, 20736):
+            for K in (128, 256, 2560, 4096, 9728):
+                assert lib.kernel(M, N, K, 1, 1) in (SPLIT, LARGE), (M, N, K)
+                others = PREVIOUS if M >= 1024 and N % 192 == 0 else SMALL
+                assert lib.kernel(M, N, K, 1, 0) in (SPLIT, others), (M, N, K)
+                assert lib.kernel(M, N, K, 0, 1) == others, (M, N, K)
+                seen |= {lib.kernel(M, N, K, 1, 1), lib.kernel(M, N, K, 1, 0)}
+            assert lib.kernel(M, N + 4, 2560, 1, 1) in (SPLIT, SMALL), (M, N + 4)  # (rows of 8 outputs)
+    assert seen == {SPLIT, LARGE, SMALL, PREVIOUS}
+
+
+def test_the_gpu_tests_reach_every_kernel(lib):
+    """The sizes of the GPU tests, by the kernel that serves them."""
+    import test_gpu_fp8_split as split
+    import test_gpu_gemm as gemm
+    by = {}
+    for size in split.SIZES:
+        for rows16 in (1, 0):  # (the padded outputs rule out 16-byte rows)
+            by.setdefault(lib.kernel(*size, 1, rows16), []).append(size)
+    assert len(by[SPLIT]) > 10
+    assert {M for M, _, _ in by[LARGE]} >= {129, 200, 239, 255, 257, 20000}
+    assert len(by[SMALL]) >= 3 and len(by[PREVIOUS]) >= 1
+    assert lib.kernel(*gemm.FP8_VARIANT_SIZE, 1, 1) == LARGE and lib.kernel(*gemm.FP8_VARIANT_SIZE, 1, 0) == PREVIOUS
+    assert lib.kernel(*gemm.FP8_SMALL_SIZE, 0, 1) == SMALL

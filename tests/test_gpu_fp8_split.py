@@ -1,4 +1,4 @@
-"""The split-K FP8 GEMM at the edges of its tiles, its K split and its dispatch range."""
+"""The FP8 GEMMs at the edges of their tiles, of the split kernel's K split and of the dispatch."""
 import pytest
 import torch
 
@@ -9,13 +9,14 @@ DEV = "cuda"
 
 
 # (M, N, K): M around 16, 32 and 64 rows; N with a part tile (and not a multiple of 4 or 16);
-# one k-step, fewer k-steps than wavefronts and splits of unequal length; the sizes around
-# which the planner hands over to the 128 x 128 tiles, and the large-tile kernel's lower end; a
-# single part tile of activation rows and of weight rows on the large tiles
+# one k-step, fewer k-steps than wavefronts and splits of unequal length, all on the split kernel;
+# one part tile of activation rows or of weight rows on the large tiles; sizes of large tiles that
+# run on 128 x 128 or on the previous 256 x 192 tiles where y's rows rule the large ones out
 SIZES = [(1, 16, 128), (1, 6144, 2560), (2, 20, 256), (15, 48, 384), (16, 2560, 9728), (17, 33, 640), (32, 80, 1152),
          (33, 6144, 2560), (49, 130, 256), (64, 1008, 1024), (65, 2560, 4096), (129, 200, 896), (255, 19456, 256),
          (257, 19456, 256), (300, 1024, 1024), (512, 6144, 640), (1023, 192, 384), (1024, 192, 384), (1025, 208, 384),
-         (65, 19456, 256), (129, 19456, 256), (200, 19456, 256), (239, 19456, 256), (20000, 128, 2560)]
+         (65, 19456, 256), (129, 17280, 384), (200, 19456, 256), (239, 19456, 256), (20000, 128, 2560),
+         (257, 16501, 640), (400, 14500, 512), (513, 11000, 512), (1300, 4800, 512)]
 
 
 @pytest.mark.parametrize("M,N,K", SIZES)

@@ -322,20 +322,26 @@ def test_w4a16_elementwise_vs_reference_formula(M, symmetric):
     assert (diff <= bound).all()
 
 
+# large tiles, and for outputs whose rows rule them out the previous 256 x 192 kernel; the 128 x 128
+# tiles where the buffer kernels are switched off (tests/test_fp8_plan.py holds both to the plan)
+FP8_VARIANT_SIZE, FP8_SMALL_SIZE = (2048, 1920, 2560), (300, 1000, 640)
+
+
 @pytest.mark.parametrize("variant", ["default", "four_waves", "previous_family", "strided_y"])
-def test_fp8_gemm_kernel_variants(variant, miq_env):
-    """Every FP8 kernel the dispatcher can reach at the large-tile shapes: the 8-wavefront
-    256x192 kernel (default), its 4-wavefront layout (MIQ_FP8_WAVES=4), the previous
-    256x192 family (MIQ_FP8_OLD, also taken for an output whose row stride is not a
-    multiple of 8), and a strided output through the C ABI (ldy = N + 4)."""
+@pytest.mark.parametrize("M,N,K", [(1024, 1920, 2560), FP8_VARIANT_SIZE, FP8_SMALL_SIZE])
+def test_fp8_gemm_kernel_variants(variant, M, N, K, miq_env):
+    """Every FP8 kernel that the dispatcher can reach besides the split one (which has the first
+    size where no switch is set): the 8-wavefront 256x192 kernel (default), its 4-wavefront
+    layout (MIQ_FP8_WAVES=4), the previous 256x192 family (MIQ_FP8_OLD, also taken for an
+    output whose row stride is not a multiple of 8) or, at the last size, the 128x128 tiles,
+    and a strided output through the C ABI (ldy = N + 4)."""
     from kernels import _lib as L
     from kernels import quant_ops as ops
-    case(f"fp8 gemm variant {variant}")
+    case(f"fp8 gemm variant {variant} M={M} N={N} K={K}")
     if variant == "four_waves":
         miq_env("MIQ_FP8_WAVES", "4")
     if variant == "previous_family":
         miq_env("MIQ_FP8_OLD", "1")
-    M, N, K = 1024, 1920, 2560
     x = torch.randn(M, K, generator=gen(54)).to(torch.bfloat16)
     w = make_w(N, K, 55)
     xq, xs = O.fp8_quantize_activation(x)
