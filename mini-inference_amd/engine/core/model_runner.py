@@ -94,6 +94,23 @@ class Request:
         return len(self.prompt_ids) + self.max_new_tokens
 
 
+def join_ints(pieces):
+    """Lists and tensors of whole numbers, in order, as one int64 tensor on the host. Neighbouring
+    lists go into one C array (a tensor per one-token list costs more than the values)."""
+    out, run = [], array("q")
+    for piece in pieces:
+        if isinstance(piece, torch.Tensor):
+            if run:
+                out.append(torch.frombuffer(run, dtype=torch.int64))
+                run = array("q")
+            out.append(piece if piece.dtype == torch.int64 and not piece.is_cuda else piece.to("cpu", torch.int64))
+        else:
+            run.extend(piece)
+    if run:
+        out.append(torch.frombuffer(run, dtype=torch.int64))
+    return out[0] if len(out) == 1 else torch.cat(out)
+
+
 class BatchMetadata:
     """What every layer of one step needs (reference model_runner.py:11-61):
 
@@ -113,20 +130,27 @@ class BatchMetadata:
         firsts = [e - n for e, n in zip(ends, lengths)]  # first row of each chunk
         is_decode = [n == 1 and start > 0 for n, (_, start, _) in zip(lengths, chunks)]
 
-        # this library's own cache hands out slots and pages as plain integers; another one is asked
-        # through its slots() and decode_tables()
+        # one token's slot and a decode row's pages come as plain integers from this library's own
+        # cache; longer chunks, and caches that answer slots() or decode_tables() themselves,
+        # give tensors (a 32768-token prompt as plain integers took twice the time)
         own = (isinstance(cache, CacheBookkeeping) and type(cache).slots is CacheBookkeeping.slots
                and type(cache).decode_tables is CacheBookkeeping.decode_tables)
-        token_ids, positions, slots = [], [], []
-        for n, (req, start, end) in zip(lengths, chunks):
+        token_ids, positions, slots, contexts = [], [[]], [[]], []
+        for n, dec, (req, start, end) in zip(lengths, is_decode, chunks):
             token_ids += req.ids(start, end) if type(req) is Request else req.all_ids[start:end]
-            positions += range(start, end)
-            slots += [cache.slot(req, start)] if n == 1 and own else cache.slots(req, start, end).tolist()
+            if not dec:
+                contexts.append(cache.slots(req, 0, end))
+            if n == 1 and own:
+                positions[-1].append(start)
+                slots[-1].append(cache.slot(req, start))
+            else:
+                positions += (torch.arange(start, end), [])
+                slots += (contexts[-1] if own and start == 0 else cache.slots(req, start, end), [])
         self.num_tokens = ends[-1] if ends else 0
         self.context_tokens = sum(end for _, _, end in chunks)
 
-        self.prefill = [(first, end - start, start, cache.slots(req, 0, end).to(device))
-                        for first, dec, (req, start, end) in zip(firsts, is_decode, chunks) if not dec]
+        prompts = [(first, n, start) for first, n, dec, (_, start, _) in zip(firsts, lengths, is_decode, chunks) if not dec]
+        self.prefill = [(*prompt, context.to(device)) for prompt, context in zip(prompts, contexts)]
         decodes = [(first, req, end) for first, dec, (req, _, end) in zip(firsts, is_decode, chunks) if dec]
         self.all_decode = not self.prefill
         self.decode_tables = None
@@ -137,15 +161,14 @@ class BatchMetadata:
         # one host buffer and one copy for everything the step indexes by: five int64 lists, then
         # the block table and the context lengths as int32 (a copy per list costs a launch and a
         # wait each)
-        parts = [token_ids, positions, slots, [e - 1 for e in ends], [row for row, _, _ in decodes]]
-        ints = array("q", itertools.chain.from_iterable(parts))
+        parts = [[token_ids], positions, slots, [[e - 1 for e in ends]], [[row for row, _, _ in decodes]]]
         flat.extend(lens)
         if len(flat) % 2:
             flat.append(0)
-        ints.frombytes(flat.tobytes())
-        held = torch.frombuffer(ints, dtype=torch.int64).to(device, copy=True) if ints else torch.empty(
-            0, dtype=torch.int64, device=device)
-        at = list(itertools.accumulate((len(p) for p in parts), initial=0))
+        words = array("q")
+        words.frombytes(flat.tobytes())
+        held = join_ints([*itertools.chain.from_iterable(parts), words]).to(device, copy=True)
+        at = list(itertools.accumulate((sum(map(len, p)) for p in parts), initial=0))
         self.input_ids, self.positions, self.write_slots, self.last_rows, self.decode_rows = (
             held[a:b] for a, b in zip(at, at[1:]))
         if paged and not own:

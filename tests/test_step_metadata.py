@@ -63,6 +63,43 @@ def test_indexes_equal_the_per_request_ones(mode, kind, starts, backend):
         assert meta.decode_tables is None
 
 
+@pytest.mark.parametrize("mode", ["paged", "contiguous"])
+def test_prompts_stay_tensors(mode, monkeypatch):
+    """The slots and positions of a prompt or a longer chunk never become Python integers (which
+    takes longer than the rest of the metadata), next to decode rows either."""
+    cache = Cache(mode)
+    chunks = [(r, s, n) for r, s, n in zip(requests(cache, [9, 30, 17, 1], seed=5), [8, 0, 5, 0], [9, 30, 17, 1])]
+
+    def refuse(tensor):
+        raise AssertionError(f"{tensor.numel()} values to Python")
+
+    with monkeypatch.context() as patch:
+        patch.setattr(torch.Tensor, "tolist", refuse)
+        meta = BatchMetadata(chunks, cache, "cpu")
+    assert torch.equal(meta.positions, torch.cat([torch.arange(s, e) for _, s, e in chunks]))
+    assert torch.equal(meta.write_slots, torch.cat([cache.slots(r, s, e) for r, s, e in chunks]))
+    for (first, n, start, context), (r, s, e) in zip(meta.prefill, chunks[1:]):
+        assert (n, start) == (e - s, s) and torch.equal(context, cache.slots(r, 0, e))
+
+
+def test_a_step_without_chunks_is_refused():
+    with pytest.raises(RuntimeError):
+        BatchMetadata([], Cache("paged"), "cpu")
+
+
+def test_slots_of_another_width_are_taken():
+    """A cache's own slots() may give 32-bit values."""
+    class Narrow(Cache):
+        def slots(self, req, start, end):
+            return super().slots(req, start, end).int()
+
+    cache = Narrow("paged")
+    chunks = [(r, s, n) for r, s, n in zip(requests(cache, [9, 30], seed=5), [8, 0], [9, 30])]
+    meta = BatchMetadata(chunks, cache, "cpu")
+    assert meta.write_slots.dtype == torch.int64
+    assert meta.write_slots.tolist() == [t for r, s, e in chunks for t in cache.slots(r, s, e).tolist()]
+
+
 def test_tables_do_not_alias_the_allocator():
     """The packed tables are copies: growing a request later leaves an older step's table alone."""
     lists = [[3, 1], [2]]
