@@ -83,7 +83,7 @@ def test_prompts_stay_tensors(mode, monkeypatch):
 
 
 def test_a_step_without_chunks_is_refused():
-    with pytest.raises(RuntimeError):
+    with pytest.raises((RuntimeError, ValueError), match="non-empty"):
         BatchMetadata([], Cache("paged"), "cpu")
 
 
