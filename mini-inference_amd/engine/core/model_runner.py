@@ -36,7 +36,8 @@ from array import array
 import torch
 import torch.nn.functional as F
 
-from engine.core.kv_cache import CacheBookkeeping, flat_block_tables, rotate_half
+from engine.core.kv_cache import (CacheBookkeeping, ContiguousAllocator, PagedAllocator, flat_block_tables,
+                                  rotate_half)
 
 SUPPORTED = ("OlmoeForCausalLM", "Qwen3ForCausalLM", "Qwen3MoeForCausalLM", "Qwen2ForCausalLM")
 _PAGED_BACKENDS = ("triton", "paged")
@@ -94,6 +95,17 @@ class Request:
         return len(self.prompt_ids) + self.max_new_tokens
 
 
+def gives_plain_integers(cache):
+    """Whether `slot` and `page_lists` of the cache stand for its slots() and decode_tables(): this
+    library's bookkeeping and allocators, with neither method replaced in a subclass or on an
+    object."""
+    kind = type(cache)
+    return (isinstance(cache, CacheBookkeeping) and kind.slots is CacheBookkeeping.slots
+            and kind.decode_tables is CacheBookkeeping.decode_tables
+            and type(cache.allocator) in (PagedAllocator, ContiguousAllocator) and "slots" not in vars(cache.allocator)
+            and "slots" not in vars(cache) and "decode_tables" not in vars(cache))
+
+
 def join_ints(pieces):
     """Lists and tensors of whole numbers, in order, as one int64 tensor on the host. Neighbouring
     lists go into one C array (a tensor per one-token list costs more than the values)."""
@@ -131,10 +143,9 @@ class BatchMetadata:
         is_decode = [n == 1 and start > 0 for n, (_, start, _) in zip(lengths, chunks)]
 
         # one token's slot and a decode row's pages come as plain integers from this library's own
-        # cache; longer chunks, and caches that answer slots() or decode_tables() themselves,
+        # allocators; longer chunks, and caches that answer slots() or decode_tables() themselves,
         # give tensors (a 32768-token prompt as plain integers took twice the time)
-        own = (isinstance(cache, CacheBookkeeping) and type(cache).slots is CacheBookkeeping.slots
-               and type(cache).decode_tables is CacheBookkeeping.decode_tables)
+        own = gives_plain_integers(cache)
         token_ids, positions, slots, contexts = [], [[]], [[]], []
         for n, dec, (req, start, end) in zip(lengths, is_decode, chunks):
             token_ids += req.ids(start, end) if type(req) is Request else req.all_ids[start:end]

@@ -100,6 +100,43 @@ def test_slots_of_another_width_are_taken():
     assert meta.write_slots.tolist() == [t for r, s, e in chunks for t in cache.slots(r, s, e).tolist()]
 
 
+@pytest.mark.parametrize("where", ["slots", "decode_tables", "allocator", "allocator_class"])
+def test_replaced_methods_are_asked(where):
+    """A slots() or decode_tables() set on the cache object, a slots() set on its allocator, and
+    an allocator of another class are used for decode rows too."""
+    cache = Cache("paged")
+    plain_slots, plain_tables = cache.slots, cache.decode_tables
+    if where == "slots":
+        cache.slots = lambda req, start, end: plain_slots(req, start, end) + 1000
+    elif where == "decode_tables":
+        cache.decode_tables = lambda entries, device: ("tables", entries, device, 7)
+    elif where == "allocator":
+        inner = cache.allocator.slots
+        cache.allocator.slots = lambda req, start, end: inner(req, start, end) + 1000
+    else:
+        class Shifted:  # (no slot(), as an allocator may lack it)
+            def __init__(self, own):
+                self.own, self.tables, self.block_size, self.blocks_for = own, own.tables, own.block_size, own.blocks_for
+
+            def __getattr__(self, name):
+                if name == "slot":
+                    raise AttributeError(name)
+                return getattr(self.own, name)
+
+            def slots(self, req, start, end):
+                return self.own.slots(req, start, end) + 1000
+
+        cache.allocator = Shifted(cache.allocator)
+    chunks = [(r, n - 1, n) for r, n in zip(requests(cache, [5, 9], seed=7), [5, 9])]
+    meta = BatchMetadata(chunks, cache, "cpu")
+    assert meta.write_slots.tolist() == [cache.slots(r, s, e).item() for r, s, e in chunks]
+    assert (int(meta.write_slots[0]) >= 1000) == (where != "decode_tables")
+    if where == "decode_tables":
+        assert meta.decode_tables[0] == "tables" and meta.decode_tables[3] == 7
+    else:
+        assert torch.equal(meta.decode_tables[0], plain_tables([(r, e) for r, _, e in chunks], "cpu")[0])
+
+
 def test_tables_do_not_alias_the_allocator():
     """The packed tables are copies: growing a request later leaves an older step's table alone."""
     lists = [[3, 1], [2]]
