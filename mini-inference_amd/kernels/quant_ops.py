@@ -184,7 +184,7 @@ def fp8_gemm(x_fp8, x_scale, w_fp8, w_scale):
 
 def fp8_linear(x, w_fp8, w_scale):
     """FP8WeightAct.linear on a native device (fp8.py:48-61) in one library call: the rows of
-    x quantized into a scratch buffer, then the GEMM. K must be a multiple of 128."""
+    x [M, K] quantized into a scratch buffer, then the GEMM. K must be a multiple of 128."""
     L.require_device(x, w_fp8, w_scale)
     x2 = _contig_rows(x)
     M, K = x2.shape
