@@ -357,7 +357,8 @@ class KVCache(CacheBookkeeping):
         """RoPE of q and k and the write of k and v: returns q rotated. q [T, heads, D], k and v
         [T, kv_heads, D], cos and sin [T, 1, D]. bf16 steps into an 8-bit cache on the device take
         one kernel (rope_kv_write, the same roundings); the rest the formula itself."""
-        if (self.kv_dtype is not None and q.is_cuda and type(self).write is KVCache.write and 0 < q.shape[0] < 65536
+        if (self.kv_dtype is not None and q.is_cuda and type(self).write is KVCache.write and "write" not in vars(self)
+                and 0 < q.shape[0] < 65536
                 and q.shape[-1] == 128 and all(t.dtype == torch.bfloat16 for t in (q, k, v, cos, sin))
                 and all(t.stride(-1) == 1 for t in (q, k, v)) and cos.stride() == sin.stride()
                 and cos.shape == sin.shape == (q.shape[0], 1, 128) and cos.stride(-1) == 1

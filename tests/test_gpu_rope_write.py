@@ -13,7 +13,8 @@ DEV = "cuda"
 def test_rope_kv_write_is_bit_exact(kind, model_dtype, T, heads, kv, strided):
     """Rotated queries, codes and scales equal the torch formula's followed by the two KV writes,
     bit for bit (bf16 and fp32 cache scales); q, k and v as slices of one projection too; rows
-    of zeros, of one huge value and of infinities take the same branches."""
+    of zeros and of one huge value, and an infinity in a query, a key and a value head (whose
+    scale is infinite and whose codes are those of x / inf and, at the infinity, of NaN)."""
     from engine.core.kv_cache import KVCache, rotate_half
     print(f"[case] rope kv write {kind} {model_dtype} T={T} heads={heads} kv={kv} strided={strided}", flush=True)
     g = torch.Generator().manual_seed(T * 100 + heads)
@@ -22,6 +23,8 @@ def test_rope_kv_write_is_bit_exact(kind, model_dtype, T, heads, kv, strided):
     qkv[0, heads] = 0
     qkv[-1, -1, 5] = 3e38
     qkv[-1, 0, 7] = float("inf")
+    qkv[T // 2, heads, 3] = float("-inf")
+    qkv[T // 2, heads + kv, 9] = float("inf")
     q, k, v = qkv.split([heads, kv, kv], dim=1)
     if not strided:
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
@@ -39,6 +42,32 @@ def test_rope_kv_write_is_bit_exact(kind, model_dtype, T, heads, kv, strided):
     for a, b in ((got.k, want.k), (got.v, want.v)):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     assert torch.equal(got.k_scale, want.k_scale) and torch.equal(got.v_scale, want.v_scale)
+
+
+def test_a_replaced_write_is_called():
+    """A write() of a subclass or set on the cache object gets k rotated and v."""
+    from engine.core.kv_cache import KVCache, rotate_half
+    print("[case] rope kv write, replaced write", flush=True)
+    calls = []
+
+    class Own(KVCache):
+        def write(self, layer, slots, k, v):
+            calls.append((k, v))
+
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(3, n, 128, generator=g).bfloat16().to(DEV) for n in (4, 2, 2))
+    ang = torch.randn(3, 1, 128, generator=g)
+    cos, sin = ang.cos().bfloat16().to(DEV), ang.sin().bfloat16().to(DEV)
+    slots = torch.tensor([4, 0, 9], device=DEV)
+    args = ("paged", 1, 2, 128, 16, torch.bfloat16, DEV, 16, 0.01, "fp8")
+    spied = KVCache(*args)
+    spied.write = lambda layer, slots, k, v: calls.append((k, v))
+    for cache in (Own(*args), spied):
+        out = cache.write_rotated(0, slots, q, k, v, cos, sin)
+        assert torch.equal(out, q * cos + rotate_half(q) * sin)
+    assert len(calls) == 2
+    for got_k, got_v in calls:
+        assert torch.equal(got_k, k * cos + rotate_half(k) * sin) and torch.equal(got_v, v)
 
 
 def test_other_forms_take_the_formula():
