@@ -250,12 +250,14 @@ int miq_moe_align(const void* topk_ids, int idx_dtype, int64_t num_pairs, int64_
  * down q: uint8 [E, H, I/2], scale/zero [E, H, I/group]; zero pointers may be NULL
  * (symmetric); topk_weights [T, k] in w_dtype (f32 / bf16 / f16, k <= 32); sorted_ids /
  * expert_ids / num_padded from miq_moe_align with block_m == 16. Workspace bytes from
- * miq_moe_workspace_bytes. out: bf16 [T, H].
+ * miq_moe_min_workspace_bytes, which every layer takes; INT8 layers of many tokens run faster
+ * with the larger miq_moe_workspace_bytes. out: bf16 [T, H].
  * Rounding follows the reference loop: gate/up and down outputs rounded to bf16, the
  * product with the routing weight (in its own dtype) rounded to bf16, and a token's
  * contributions added in ascending expert order with a bf16 rounding after each
  * addition (index_add_ into a bf16 output). */
 size_t miq_moe_workspace_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I);
+size_t miq_moe_min_workspace_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I);
 int miq_w4a16_moe(const void* hidden, int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk,
                   const uint8_t* gu_q, const void* gu_scale, const void* gu_zero,
                   const uint8_t* dn_q, const void* dn_scale, const void* dn_zero,
@@ -287,7 +289,7 @@ int miq_w8a16_moe(const void* hidden, int64_t T, int64_t H, int64_t I, int64_t E
  * gate_up q: e4m3fn bytes [E, 2I, H], scale fp32 [E, 2I]; down q: e4m3fn bytes [E, H, I],
  * scale fp32 [E, H]. H and I multiples of 128 and at most 4096; sorted_ids / expert_ids /
  * num_padded from miq_moe_align with block_m == 16; workspace from
- * miq_moe_workspace_bytes. out: bf16 [T, H]. */
+ * miq_moe_min_workspace_bytes. out: bf16 [T, H]. */
 int miq_fp8_moe(const void* hidden, int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk,
                 const uint8_t* gu_q, const float* gu_scale, const uint8_t* dn_q, const float* dn_scale,
                 const void* topk_weights, int w_dtype, const int32_t* sorted_ids,
@@ -299,8 +301,8 @@ int miq_fp8_moe(const void* hidden, int64_t T, int64_t H, int64_t I, int64_t E, 
  * kernels/fused_moe/fused_moe_triton.py:110-121, moe_align.cu:5-88). Up to 1024 pairs and
  * 256 experts (and, for int4, H a multiple of 128 and I of 64) the expert GEMMs form
  * moe_align's layout in LDS and no align launch runs; otherwise miq_moe_align runs into the
- * workspace. Same results as miq_moe_align followed by the layer above; same workspace
- * size (miq_moe_workspace_bytes). */
+ * workspace, or for INT8 layers of many tokens a grouping of their own. Same results as
+ * miq_moe_align followed by the layer above; same workspace sizes. */
 int miq_w4a16_moe_routed(const void* hidden, int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk,
                          const uint8_t* gu_q, const void* gu_scale, const void* gu_zero,
                          const uint8_t* dn_q, const void* dn_scale, const void* dn_zero,

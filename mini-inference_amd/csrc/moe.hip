@@ -1380,6 +1380,10 @@ size_t moe_stream_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I
 }
 }  // namespace
 
+extern "C" size_t miq_moe_min_workspace_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
+  return moe_stream_bytes(T, topk, E, H, I);
+}
+
 extern "C" size_t miq_moe_workspace_bytes(int64_t T, int64_t topk, int64_t E, int64_t H, int64_t I) {
   const size_t bytes = moe_stream_bytes(T, topk, E, H, I);
   return moe_block_ok(KIND_INT8, T, topk, E, H, I) ? std::max(bytes, moe_block_bytes(T, topk, E, H, I)) : bytes;

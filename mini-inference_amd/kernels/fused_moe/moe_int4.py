@@ -57,7 +57,7 @@ def fused_moe_int4(hidden, topk_ids, topk_weights, gu_q, gu_scale, gu_zero, dn_q
         raise RuntimeError("fused_moe_int4: gate_up and down must share one group size")
     h = hidden.contiguous()
     w = topk_weights.contiguous()  # used in its own dtype, as the reference multiplies by it
-    nbytes = L.load().miq_moe_workspace_bytes(T, k, E, H, inter)
+    nbytes = L.load().miq_moe_min_workspace_bytes(T, k, E, H, inter)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=hidden.device)
     out = torch.empty((T, H), dtype=torch.bfloat16, device=hidden.device)
     sdt = gu_scale.dtype
@@ -124,7 +124,7 @@ def fused_moe_fp8(hidden, topk_ids, topk_weights, gu_q, gu_scale, dn_q, dn_scale
         raise RuntimeError("fused_moe_fp8: scales must be float32")
     h = hidden.contiguous()
     w = topk_weights.contiguous()
-    nbytes = L.load().miq_moe_workspace_bytes(T, k, E, H, inter)
+    nbytes = L.load().miq_moe_min_workspace_bytes(T, k, E, H, inter)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=hidden.device)
     out = torch.empty((T, H), dtype=torch.bfloat16, device=hidden.device)
     weights = (L.ptr(gu_q.contiguous()), L.ptr(gu_scale.contiguous()), L.ptr(dn_q.contiguous()),

@@ -60,6 +60,20 @@ def test_workspace_sizes():
     assert lib.miq_moe_workspace_bytes(64, 8, 64, 2048, 1024) >= 64 * 8 * 2048 * 4
 
 
+def test_moe_workspace_of_each_format():
+    """INT8 layers of many tokens get the block GEMMs' share; the least that a layer takes, which
+    is what INT4 and FP8 layers use, has none of it."""
+    from kernels import _lib
+    lib = _lib.load()
+    T, k, E, H, inter = 1000, 8, 64, 2048, 1024
+    rows = T * k + E * 15  # 16-row tiles per expert
+    least = lib.miq_moe_min_workspace_bytes(T, k, E, H, inter)
+    tables = 4 * (T * k + rows + (rows + 15) // 16)
+    assert 2 * (rows * inter + T * k * H) + tables <= least <= 2 * (rows * inter + T * k * H) + tables + 6 * 256
+    assert lib.miq_moe_workspace_bytes(T, k, E, H, inter) > least
+    assert lib.miq_moe_workspace_bytes(8, k, E, H, inter) == lib.miq_moe_min_workspace_bytes(8, k, E, H, inter)
+
+
 @pytest.mark.parametrize("T,k,E", [(4, 2, 0), (0, 2, 8), (0, 0, 0), (300, 2, 0)])
 def test_workspace_query_of_empty_layers(T, k, E):
     """A layer without experts or tokens has a size too (the layer itself refuses it)."""
