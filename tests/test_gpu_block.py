@@ -10,10 +10,11 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-# M below, at and past one half block (128 rows), one block (256) and two; N with part blocks of
+# M of one row and of one 32-row fragment and one more (with the prefill kernels' own limit of 65 rows
+# lowered), below, at and past one half block (128 rows), one block (256) and two; N with part blocks of
 # 256 and part wavefronts of 64; K of two, four and ten stages; 130 blocks (a last round that is
 # not halved would need more than 256) and 260 (one full round and four halved blocks)
-LINEAR = [(1, 16, 128), (65, 48, 128), (128, 256, 256), (129, 272, 640), (255, 512, 128), (256, 64, 256),
+LINEAR = [(1, 16, 128), (33, 272, 640), (65, 48, 128), (128, 256, 256), (129, 272, 640), (255, 512, 128), (256, 64, 256),
           (257, 528, 128), (600, 1040, 640), (300, 16640, 128), (1030, 13312, 128)]
 
 
@@ -26,6 +27,7 @@ def test_w8a16_block(M, N, K, sdt, miq_env):
     at strides that take and that rule out 16-byte stores; the padding stays untouched."""
     from kernels import _lib as L
     miq_env("MIQ_WO_BLOCK", "1")
+    miq_env("MIQ_WO_PREFILL_MIN_M", "1")
     print(f"[case] w8a16 block M={M} N={N} K={K} {sdt}", flush=True)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     x = torch.randn(M, K + 8, generator=g, device=DEV).bfloat16()
