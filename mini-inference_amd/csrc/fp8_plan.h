@@ -21,12 +21,17 @@ constexpr int kFp8Outside = 0x7ffffff0;
 // taking row l / 4 and 16-byte chunk (l & 3) ^ ((l >> 4) & 3) of its load.
 constexpr int kFp8LoadRows = 16;
 
+// Whether tiles of `tile` rows cover an operand of `rows` rows without rows past its end. The scalar
+// offset of such an operand's loads may hold the load's row (q * kFp8LoadRows * K): it stays inside
+// the buffer, and so does its sum with the vector offset of load 0.
+MIQ_PLAN_FN bool fp8_whole_tiles(int rows, int tile) { return rows % tile == 0; }
+
 // Vector offset of one lane's part of load `q` of a tile that begins at row `row0`, in an operand of
 // `rows` rows of K bytes; the stage's k (a multiple of 64 below K) is the scalar offset. The row is
-// in the vector offset so that the rows past the end, which a tile has whenever its height does
-// not divide `rows`, are outside the buffer on their own: with the row in the scalar offset the
-// hardware compares the vector offset with (size - scalar offset), which is negative, and as an
-// unsigned number huge, once the tile's last rows lie more than `rows` rows into it.
+// in the vector offset so that the rows past the end of an operand that its tiles do not cover
+// evenly are outside the buffer on their own: with the row in the scalar offset the hardware
+// compares the vector offset with (size - scalar offset), which is negative, and as an unsigned
+// number huge, once the tile's last rows lie more than `rows` rows into it.
 MIQ_PLAN_FN int fp8_large_offset(int row0, int q, int lane, int rows, int K) {
   const int row = row0 + q * kFp8LoadRows + (lane >> 2);
   return row < rows ? row * K + (((lane & 3) ^ ((lane >> 4) & 3)) << 4) : kFp8Outside;

@@ -24,7 +24,7 @@ static bool through(Load l, uint32_t size, int rule) {
 
 // Lanes of the last tile's loads (`loads` loads of 16 rows) that any rule lets read past the
 // operand, that any rule rejects though their row exists, or that read another address than
-// their row and chunk. `split`: the row in the scalar offset, the k in the vector offset.
+// their row and chunk. `split`: the load's row in the scalar offset, the k in the vector offset.
 extern "C" long faults(int rows, int K, int tile, int loads, int split) {
   const uint32_t size = (uint32_t)rows * (uint32_t)K;
   const int row0 = (rows - 1) / tile * tile;
@@ -34,7 +34,7 @@ extern "C" long faults(int rows, int K, int tile, int loads, int split) {
       for (int lane = 0; lane < 64; ++lane) {
         const int row = row0 + 16 * q + lane / 4, chunk = (lane & 3) ^ ((lane >> 4) & 3);
         Load l{(uint32_t)fp8_large_offset(row0, q, lane, rows, K), (uint32_t)k0};
-        if (split) l = Load{(uint32_t)((row0 + lane / 4) * K + chunk * 16 + k0), (uint32_t)(16 * q * K)};
+        if (split) l = Load{(uint32_t)(fp8_large_offset(row0, 0, lane, rows, K) + k0), (uint32_t)(16 * q * K)};
         for (int rule = 0; rule < 3; ++rule) {
           const bool reads = through(l, size, rule);
           const uint64_t at = (uint64_t)l.voff + l.soff;
@@ -45,6 +45,8 @@ extern "C" long faults(int rows, int K, int tile, int loads, int split) {
       }
   return bad;
 }
+
+extern "C" int whole(int rows, int tile) { return fp8_whole_tiles(rows, tile); }
 
 extern "C" int kernel(long M, long N, long K, int buffers, int rows16) {
   return (int)fp8_plan(M, N, K, buffers, rows16).kernel;
@@ -85,11 +87,15 @@ def test_large_tiles_read_inside_their_operands(lib, tile, loads):
 
 
 @pytest.mark.parametrize("tile,loads", TILES)
-def test_the_check_finds_rows_in_the_scalar_offset(lib, tile, loads):
-    """The same check refuses offsets with the row in the scalar part, for operands lower than a
-    tile (a planted mistake)."""
-    for rows in (1, 65, 129, 175):
-        assert lib.faults(rows, 2560, tile, loads, 1) > 0, rows
+def test_rows_go_into_the_scalar_offset_only_with_whole_tiles(lib, tile, loads):
+    """Operands of whole tiles may have the row in the scalar part, up to the largest one; the
+    check refuses that for every other number of rows, which the rule keeps from it."""
+    for tiles in (1, 2, 11):
+        assert lib.whole(tiles * tile, tile) and lib.faults(tiles * tile, 2560, tile, loads, 1) == 0
+    last = 0x7fffff00 // 128 // tile * tile
+    assert lib.whole(last, tile) and lib.faults(last, 128, tile, loads, 1) == 0
+    for rows in (1, 65, 129, 175, tile - 1, tile + 1, 5 * tile + 64):
+        assert not lib.whole(rows, tile) and lib.faults(rows, 2560, tile, loads, 1) > 0, rows
 
 
 # (M, N, K) -> the kernel that measures fastest there, of every size by more than 5 %
