@@ -137,32 +137,30 @@ class BatchMetadata:
     """
 
     def __init__(self, chunks, cache, device, attn_backend="triton"):
-        lengths = [end - start for _, start, end in chunks]
-        ends = list(itertools.accumulate(lengths))       # row after each chunk
-        firsts = [e - n for e, n in zip(ends, lengths)]  # first row of each chunk
-        is_decode = [n == 1 and start > 0 for n, (_, start, _) in zip(lengths, chunks)]
-
         # one token's slot and a decode row's pages come as plain integers from this library's own
         # allocators; longer chunks, and caches that answer slots() or decode_tables() themselves,
         # give tensors (a 32768-token prompt as plain integers took twice the time)
         own = gives_plain_integers(cache)
-        token_ids, positions, slots, contexts = [], [[]], [[]], []
-        for n, dec, (req, start, end) in zip(lengths, is_decode, chunks):
+        token_ids, positions, slots, last_rows = [], [[]], [[]], []
+        self.prefill, decodes, first = [], [], 0
+        for req, start, end in chunks:
+            n, context = end - start, None
             token_ids += req.ids(start, end) if type(req) is Request else req.all_ids[start:end]
-            if not dec:
-                contexts.append(cache.slots(req, 0, end))
+            if n == 1 and start > 0:
+                decodes.append((first, req, end))
+            else:
+                context = cache.slots(req, 0, end)
+                self.prefill.append((first, n, start, context.to(device)))
             if n == 1 and own:
                 positions[-1].append(start)
                 slots[-1].append(cache.slot(req, start))
             else:
                 positions += (torch.arange(start, end), [])
-                slots += (contexts[-1] if own and start == 0 else cache.slots(req, start, end), [])
-        self.num_tokens = ends[-1] if ends else 0
+                slots += (context if own and start == 0 else cache.slots(req, start, end), [])
+            first += n
+            last_rows.append(first - 1)
+        self.num_tokens = first
         self.context_tokens = sum(end for _, _, end in chunks)
-
-        prompts = [(first, n, start) for first, n, dec, (_, start, _) in zip(firsts, lengths, is_decode, chunks) if not dec]
-        self.prefill = [(*prompt, context.to(device)) for prompt, context in zip(prompts, contexts)]
-        decodes = [(first, req, end) for first, dec, (req, _, end) in zip(firsts, is_decode, chunks) if dec]
         self.all_decode = not self.prefill
         self.decode_tables = None
         paged = decodes and attn_backend in _PAGED_BACKENDS
@@ -172,7 +170,7 @@ class BatchMetadata:
         # one host buffer and one copy for everything the step indexes by: five int64 lists, then
         # the block table and the context lengths as int32 (a copy per list costs a launch and a
         # wait each)
-        parts = [[token_ids], positions, slots, [[e - 1 for e in ends]], [[row for row, _, _ in decodes]]]
+        parts = [[token_ids], positions, slots, [last_rows], [[row for row, _, _ in decodes]]]
         flat.extend(lens)
         if len(flat) % 2:
             flat.append(0)
