@@ -1084,7 +1084,11 @@ void launch_stream_mode(const MoeParams& p, int grid, size_t lds, int blocks, in
 // One GEMM of the layer: NW = 8 wavefronts (twice the weight rows per staged activation
 // tile, four wavefronts per SIMD) where the sizes divide and two such workgroups fit a CU's
 // LDS, else 4; int4 with 16-bit scales keeps the item's scales in registers where a row's
-// groups fit. MIQ_MOE_WAVES=4 forces four wavefronts.
+// groups fit. With zero points and groups of 128, up to 128 items leave CUs idle on eight, and four
+// finish sooner (gate/up and down of one layer, eight / four wavefronts: 40 experts, top 3, 1536 x 512,
+// T = 1 25.0/23.4, 8 26.9/25.7, 16 27.0/27.2, 64 28.5/30.6 us; 16, top 4, 1024 x 512, T = 64
+// 24.9/24.0, 128 26.0/28.6); groups of 256 go either way (0.93 to 1.07) and stay on eight.
+// MIQ_MOE_WAVES=4 forces four wavefronts.
 template <int KIND, int MODE, bool HZ, int SD, bool G1>
 void launch_stream_gemm(const MoeParams& p, int max_tiles, hipStream_t st) {
   const size_t lds = KIND == KIND_FP8 ? (size_t)kTile * kF8Row + (size_t)kF8Steps * kTile * 4
@@ -1095,7 +1099,10 @@ void launch_stream_gemm(const MoeParams& p, int max_tiles, hipStream_t st) {
   const bool sl = kSL16 && ng % 4 == 0 && ng <= kMoeRegGroups && !tuning().moe_no_lds_scales;
   const int per8 = MODE == MOE_GU ? 16 * 8 : 32 * 8;  // weight columns / rows of an 8-wavefront item
   const int nout = MODE == MOE_GU ? p.I : p.H;
-  const bool w8 = !tuning().moe_four_waves && nout % per8 == 0 &&
+  // (an estimate: the pairs' experts are known to the device only)
+  const int likely_tiles = std::min(p.num_pairs, p.E) + p.num_pairs / kTile;
+  const bool few = HZ && G1 && sl && likely_tiles * (nout / per8) <= 128;
+  const bool w8 = !tuning().moe_four_waves && nout % per8 == 0 && !few &&
                   2 * (lds + kMoeStaticLds) <= (size_t)160 * 1024;
   const int blocks = nout / (w8 ? per8 : per8 / 2);
   // about two workgroups per CU, never more than the runs of items that could exist

@@ -17,10 +17,12 @@ def _routed(T, H, E, k, seed):
     return hidden, w.to(torch.bfloat16), idx
 
 
-@pytest.mark.parametrize("T,H,I,E,k", [(20, 1536, 512, 4, 2), (17, 512, 1536, 5, 2), (16, 2048, 2048, 3, 1)])
+@pytest.mark.parametrize("T,H,I,E,k", [(20, 1536, 512, 4, 2), (17, 512, 1536, 5, 2), (16, 2048, 2048, 3, 1),
+                                       (400, 1536, 512, 4, 2), (300, 512, 1536, 5, 2), (200, 2048, 2048, 3, 1)])
 @pytest.mark.parametrize("sym", [False, True])
 def test_int4_scales_from_registers(T, H, I, E, k, sym):
-    """Rows of 4, 12 and 16 groups in eight-wavefront workgroups: every group's scale (and
+    """Rows of 4, 12 and 16 groups in four-wavefront workgroups (few tokens, with zero points) and
+    in eight-wavefront ones: every group's scale (and
     zero) word comes from the lane that loaded it. The groups' scales differ by powers of
     two, so a word taken from a wrong lane or slot moves the output far past the bound,
     which is the fused INT4 layer's (fp32 sums in another order, bf16 roundings alike)."""
