@@ -400,9 +400,12 @@ bool fits(int64_t M, int64_t N, int64_t K, int64_t ldx) {
 //     .. 1.33), by 8 to 37 % (19456 x 2560 M = 1024 / 2048 109 / 187 against 130 / 249 us, ratio
 //     1.02 / 0.90; 6144 x 2560 M = 1536 56 / 68, 1.29; 4096 x 12288 M = 3000 262 / 284, 1.24);
 //   one row tile or K splits: faster or even up to 1.13 (6144 x 2560 M = 512 34 / 37, 1.13; 2560 x
-//     9728 M = 2048 111 / 135, 0.99; 4096 x 12288 M = 1280 139 / 162, 1.07; 2560 x 4096 M = 1024
-//     47 / 47, 1.10), slower from 1.15 up (12288 x 4096 M = 256 50 / 47, 1.15; 2560 x 9728 M = 1536
-//     / 1024 106 / 101, 1.32, and 103 / 77, 1.77).
+//     9728 M = 2048 111 / 135, 0.99; 4096 x 12288 M = 1280 139 / 162, 1.07), slower from 1.15 up
+//     (12288 x 4096 M = 256 50 / 47, 1.15; 2560 x 9728 M = 1536 / 1024 106 / 101, 1.32, and 103 / 77,
+//     1.77);
+//   one row tile at a deep K: even at 1.07, slower from there (a second sweep of nine N, seven K and 22
+//     M: at K = 2560 the block took 0.85 to 0.98 of the wide kernel's time up to 1.14, at K = 4096
+//     0.85 to 0.94 up to 1.06 and 0.92 to 1.08 past it; 6144 x 4096 M = 450 47.8 / 45.0, 1.14).
 bool wo_block_planned(int64_t M, int64_t N, int64_t K, int64_t ldx, const WidePlan& wide) {
   const Tuning& t = tuning();
   if (t.wo_block == 0 || !fits(M, N, K, ldx)) return false;
@@ -413,7 +416,8 @@ bool wo_block_planned(int64_t M, int64_t N, int64_t K, int64_t ldx, const WidePl
   const int64_t units = 2 * (T / 256) + (rest == 0 ? 0 : rest <= 128 ? 1 : 2);
   const double block_us = 4.0 + 0.83 * (double)(units * (K / kBK));
   const double wide_us = wide.us + 4.0 + 0.35e-6 * (double)wide.pack_bytes;
-  return block_us < (wide.S == 1 && wide.mt >= 2 ? 1.35 : 1.14) * wide_us;
+  const double line = wide.S == 1 && wide.mt >= 2 ? 1.35 : wide.S == 1 && K >= 3584 ? 1.06 : 1.14;
+  return block_us < line * wide_us;
 }
 
 int wo_block_launch(const uint16_t* x, int64_t ldx, const uint8_t* w, const void* scale, int sd, uint16_t* y, int64_t ldy,

@@ -45,7 +45,8 @@ def test_w8a16_block(M, N, K, sdt, miq_env):
         assert (y[:, N:] == 7.0).all()
 
 
-@pytest.mark.parametrize("M,N,K,block", [(2048, 19456, 2560, True), (1000, 6144, 2560, True), (200, 2560, 9728, False)])
+@pytest.mark.parametrize("M,N,K,block", [(2048, 19456, 2560, True), (1000, 6144, 2560, True), (200, 2560, 9728, False),
+                                         (450, 6144, 4096, False), (512, 6144, 2560, True)])
 def test_w8a16_block_is_the_planned_kernel(M, N, K, block, miq_env):
     """The dispatch rule on both sides of its line: the call gives the bytes of the kernel that
     the rule names."""
