@@ -51,8 +51,6 @@ constexpr int kStageBytes = kXBytes<WM> + 64 * (8 / WM) * 64;
 constexpr int kOutB = 0x7f000000;             // outside every buffer, also with a k offset added
 constexpr int kBlkThreads = 512;
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
 
 struct BlockParams {
   const uint16_t* x;
@@ -79,19 +77,6 @@ struct BlockParams {
 template <int N>
 __device__ inline void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// 8 int8 codes -> 8 bf16 (exact)
-__device__ inline bf16x8 bf16_of_i8(uint32_t a, uint32_t b) {
-  auto two = [](int lo, int hi) {
-    const bf16x2_t v = {static_cast<__bf16>(static_cast<float>(lo)), static_cast<__bf16>(static_cast<float>(hi))};
-    return __builtin_bit_cast(uint32_t, v);
-  };
-  const uint4 o = make_uint4(two(static_cast<int8_t>(a), static_cast<int8_t>(a >> 8)),
-                             two(static_cast<int8_t>(a >> 16), static_cast<int8_t>(a >> 24)),
-                             two(static_cast<int8_t>(b), static_cast<int8_t>(b >> 8)),
-                             two(static_cast<int8_t>(b >> 16), static_cast<int8_t>(b >> 24)));
-  return __builtin_bit_cast(bf16x8, o);
 }
 
 __device__ inline float bf16r(float f) { return bf16_to_f32(f32_to_bf16(f)); }

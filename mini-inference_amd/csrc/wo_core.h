@@ -27,6 +27,8 @@
 namespace miq {
 namespace wo {
 
+typedef __attribute__((address_space(3))) void* lds_ptr;  // of loads that go straight to LDS
+
 constexpr int kStepK = 128;
 enum { KIND_INT8 = 0, KIND_INT4 = 1 };
 
@@ -53,6 +55,19 @@ __device__ inline bf16x8 unpack_u4(uint32_t w) {
   asm("" : "=s"(m) : "0"(0x000f000fu));
   asm("" : "=v"(o) : "0"(0x43004300u));
   return as_bf16x8((w & m) | o, ((w >> 4) & m) | o, ((w >> 8) & m) | o, ((w >> 12) & m) | o);
+}
+
+// 8 int8 codes -> 8 bf16 (exact)
+__device__ inline bf16x8 bf16_of_i8(uint32_t a, uint32_t b) {
+  auto two = [](int lo, int hi) {
+    typedef __bf16 pair __attribute__((ext_vector_type(2)));
+    const pair v = {static_cast<__bf16>(static_cast<float>(lo)), static_cast<__bf16>(static_cast<float>(hi))};
+    return __builtin_bit_cast(uint32_t, v);
+  };
+  return as_bf16x8(two(static_cast<int8_t>(a), static_cast<int8_t>(a >> 8)),
+                   two(static_cast<int8_t>(a >> 16), static_cast<int8_t>(a >> 24)),
+                   two(static_cast<int8_t>(b), static_cast<int8_t>(b >> 8)),
+                   two(static_cast<int8_t>(b >> 16), static_cast<int8_t>(b >> 24)));
 }
 
 // 4 int8 codes -> 2 dwords of bf16 (128 + q), natural order. The integers 0..255 are

@@ -40,21 +40,6 @@ struct WoSplitParams {
   bool vec_store;  // y rows 8-byte aligned (4 outputs per store)
 };
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
-
-// 8 int8 codes -> 8 bf16 (exact)
-__device__ inline bf16x8 bf16_of_i8(uint32_t a, uint32_t b) {
-  auto two = [](int lo, int hi) {
-    const bf16x2_t v = {static_cast<__bf16>(static_cast<float>(lo)), static_cast<__bf16>(static_cast<float>(hi))};
-    return __builtin_bit_cast(uint32_t, v);
-  };
-  const uint4 o = make_uint4(two(static_cast<int8_t>(a), static_cast<int8_t>(a >> 8)),
-                             two(static_cast<int8_t>(a >> 16), static_cast<int8_t>(a >> 24)),
-                             two(static_cast<int8_t>(b), static_cast<int8_t>(b >> 8)),
-                             two(static_cast<int8_t>(b >> 16), static_cast<int8_t>(b >> 24)));
-  return __builtin_bit_cast(bf16x8, o);
-}
 
 // f(integral_constant 0) .. f(integral_constant kAhead - 1)
 template <int I = 0, class F>
