@@ -65,12 +65,13 @@ class FP8WeightAct(QuantMethod):
     def linear(self, x, qweight, scale):
         """fp8.py:48-73."""
         out_dtype = x.dtype
-        x2d = x.reshape(-1, x.shape[-1])
-        K = x2d.shape[-1]
-        own_quantize = type(self).quantize_activation is FP8WeightAct.quantize_activation
-        if self.native and K % 128 == 0 and x2d.shape[0] > 0 and own_quantize and "quantize_activation" not in vars(self):
+        K = x.shape[-1]
+        x2d = x if x.dim() == 2 else x.reshape(-1, K)
+        if (self.native and K % 128 == 0 and x2d.shape[0] > 0
+                and self.quantize_activation is FP8WeightAct.quantize_activation):
             # quantize + GEMM in one library call (two calls cost twice the host time: a decode
-            # batch's linear took 29 us per call with the GPU busy for 10)
+            # batch's linear took 29 us per call with the GPU busy for 10); one replaced in a
+            # subclass or on the object is called below
             y = ops.fp8_linear(x2d, qweight, scale).to(out_dtype)
             return y if x.dim() == 2 else y.reshape(*x.shape[:-1], -1)
         x_fp8, x_scale = self.quantize_activation(x2d)
